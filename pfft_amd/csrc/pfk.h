@@ -124,7 +124,7 @@ typedef struct pfk_pass {
    * inner FFT of about the line's own length between elementwise pre and
    * post steps (pfk_r2r_inner), through `work` and `work2` */
   int32_t r2r_path;
-  int32_t pad3;
+  int32_t cache;      /* PFK_KEEP_*: accesses that leave the data in the memory-side cache */
   /* device twiddle tables (owned by the host plan):
    *   tw  : W_nf^m = exp(sign*2*pi*i*m/nf), m in [0,nf)
    *   rtw : W_n^k  = exp(sign*2*pi*i*k/n),  k in [0,n/2] (even r2c/c2r only) */
@@ -133,6 +133,12 @@ typedef struct pfk_pass {
   /* element counts of the src/dst buffers, for host-side bounds checks */
   int64_t src_elems, dst_elems;
 } pfk_pass;
+
+/* pfk_pass.cache: the source is read / the destination written with ordinary
+ * accesses, which leave the lines in the 256 MB memory-side cache, instead
+ * of streaming ones.  Kernels without streaming accesses ignore it. */
+#define PFK_KEEP_SRC 1
+#define PFK_KEEP_DST 2
 
 /* Longest computed line one workgroup transforms. */
 #define PFK_MAXLINE 4096
