@@ -826,6 +826,9 @@ int pfk_r2r_inner(const pfk_pass *p, pfk_pass *in, int64_t *ld1, int64_t *ld2, i
   in->prec = p->prec;
   in->xcd_remap = p->xcd_remap;
   in->tw = p->tw;
+  in->mix_n = p->mix_n;
+  memcpy(in->mix_rad, p->mix_rad, sizeof in->mix_rad);
+  in->twm = p->twm;
   in->text = lines;
   in->nb = 0;
   if (even) {
@@ -875,7 +878,9 @@ int pfk_r2r_inner(const pfk_pass *p, pfk_pass *in, int64_t *ld1, int64_t *ld2, i
 
 int pfk_pass_check(const pfk_pass *p) {
   if (pfk_init()) return 1;
-  if (!g_generic_only && (fast_covers(p) || small_covers(p) || mfma_covers(p))) return 0;
+  if (!g_generic_only &&
+      (fast_covers(p) || small_covers(p) || mfma_covers(p) || mixed_covers(p)))
+    return 0;
   int C, pitch;
   size_t lds;
   return generic_tiling(p, &C, &pitch, &lds);
@@ -890,12 +895,15 @@ int pfk_launch_pass(const pfk_pass *p, const void *src, void *dst) {
     if (m == 0) return 0;
     if (m < 0) return 1;
   }
-  // variant 1: general kernel; 3: short-length kernel first where it has
-  // one; else the power-of-two kernels, then the short-length kernels
+  // variant 1: general kernel; 3, 9: short-length / mixed-radix kernel first
+  // where it has one; else the power-of-two kernels, then the short-length
+  // and the mixed-radix kernels
   int r = 1;
   if (!g_generic_only && p->variant == 3) r = launch_small(p, src, dst);
+  if (!g_generic_only && p->variant == 9) r = launch_mixed(p, src, dst);
   if (r > 0) r = launch_fast(p, src, dst);
   if (r > 0 && !g_generic_only && p->variant != 1) r = launch_small(p, src, dst);
+  if (r > 0 && !g_generic_only && p->variant != 1) r = launch_mixed(p, src, dst);
   if (r == 0) return 0;
   if (r < 0) return 1;
   return launch_generic(p, src, dst);

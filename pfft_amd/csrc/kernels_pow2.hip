@@ -115,5 +115,6 @@ extern "C" int pfk_pass_kernels(const pfk_pass *p) {
   if (pfk::mfma_covers(p)) m |= PFK_HAS_MFMA;
   if (pfk::fast_covers(p)) m |= PFK_HAS_POW2;
   if (pfk::small_covers(p)) m |= PFK_HAS_SMALL;
+  if (pfk::mixed_covers(p)) m |= PFK_HAS_MIXED;
   return m;
 }

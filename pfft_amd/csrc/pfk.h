@@ -43,6 +43,7 @@ extern "C" {
 
 #define PFK_MAXB 6
 #define PFK_MAXSTAGES 24
+#define PFK_MIX_MAXST 7   /* stages of the mixed-radix kernel */
 
 enum pfk_kind { PFK_C2C = 0, PFK_R2C = 1, PFK_C2R = 2, PFK_COPY = 3, PFK_R2R = 4 };
 
@@ -96,9 +97,9 @@ typedef struct pfk_pass {
   int32_t xcd_remap;  /* map consecutive tiles to one XCD (see kernels_pow2.hip) */
   int32_t mfma;       /* complex64 c2c arithmetic form: 0 plain, 1 FP32 MFMA, 2 split-BF16 MFMA */
   int32_t variant;    /* launch variant: 0 default, 1 general kernel, 2 narrow power-of-two
-                         tiles, 3 short-length register kernel; + 4 (with 0 or 2): one
-                         workgroup per tile instead of the persistent grid; + 8: line-major
-                         lane order (complex64 c2c) */
+                         tiles, 3 short-length register kernel, 9 mixed-radix kernel; + 4
+                         (with 0 or 2): one workgroup per tile instead of the persistent
+                         grid; + 8 (with 0, 2, 4, 6): line-major lane order */
   int32_t r2r;        /* enum pfk_r2r of a PFK_R2R pass */
   /* Long lines (nf > PFK_MAXLINE): nf = n1 * n2 is computed in two
    * steps through `work` (lines * nf complex elements, owned by the plan):
@@ -130,6 +131,13 @@ typedef struct pfk_pass {
    *   rtw : W_n^k  = exp(sign*2*pi*i*k/n),  k in [0,n/2] (even r2c/c2r only) */
   const void *tw;
   const void *rtw;
+  /* mixed-radix kernel (pfk_mix_factorize): stage count (0: none), radices
+   * and the forward twiddles in stage order: for stage s > 0 with L the
+   * product of the earlier radices, W_(L R)^(r k) at [(r-1) L + k], r in
+   * [1, R), k in [0, L), and behind them, for a radix above 16, W_R^m, m < R */
+  int32_t mix_n;
+  int32_t mix_rad[PFK_MIX_MAXST];
+  const void *twm;
   /* element counts of the src/dst buffers, for host-side bounds checks */
   int64_t src_elems, dst_elems;
 } pfk_pass;
@@ -153,6 +161,56 @@ static inline int pfk_factorize(int64_t nf, int32_t *radix) {
   for (int64_t q = 3; m > 1 && ns < PFK_MAXSTAGES; q += 2)
     while (m % q == 0 && ns < PFK_MAXSTAGES) { radix[ns++] = (int32_t)q; m /= q; }
   return m == 1 ? ns : -1;
+}
+
+/* Radices of the mixed-radix kernel for length nf.  Prime factors above 13
+ * come first, a stage each (matrix cores); the rest is split into radices from
+ * 2..16: the fewest stages, and among those the smallest largest
+ * radix (fewest registers).  The first is the largest odd one, else the
+ * largest that is 2 mod 4 (its stores to LDS then meet no bank twice), the
+ * others follow in descending order.  Returns the stage count, 0 if there are
+ * more than PFK_MIX_MAXST. */
+static inline int pfk_mix_search(int64_t m, int maxr, int left, int32_t *out) {
+  if (m == 1) return 1;
+  if (left == 0) return 0;
+  for (int r = maxr; r >= 2; r--)
+    if (m % r == 0) {
+      out[0] = r;
+      if (pfk_mix_search(m / r, r, left - 1, out + 1)) return 1;
+    }
+  return 0;
+}
+static inline int pfk_mix_factorize(int64_t nf, int32_t *rad) {
+  int big = 0;
+  int64_t rest = 1, m = nf;
+  for (int64_t q = 2; m > 1; q++) {   /* primes in ascending order */
+    if (q * q > m) q = m;
+    for (; m % q == 0; m /= q) {
+      if (q <= 13) {
+        rest *= q;
+      } else {
+        if (big == PFK_MIX_MAXST) return 0;
+        rad[big++] = (int32_t)q;
+      }
+    }
+  }
+  if (rest == 1) return big;
+  for (int n = 1; rest > 1 && n <= PFK_MIX_MAXST - big; n++)
+    for (int maxr = 2; maxr <= 16; maxr++)
+      if (pfk_mix_search(rest, maxr, n, rad + big)) {
+        int32_t *r = rad + big;
+        int k = 0, f = 0;
+        for (int64_t m = rest; m > 1; k++) m /= r[k];
+        while (f < k && r[f] % 2 == 0) f++;
+        if (f == k) for (f = 0; f < k && r[f] % 4 != 2; f++) { }
+        if (f < k) {
+          const int32_t r0 = r[f];
+          for (; f > 0; f--) r[f] = r[f - 1];
+          r[0] = r0;
+        }
+        return big + k;
+      }
+  return 0;
 }
 
 /* Split of a long computed length nf = n1 * n2 with both factors at most
@@ -277,11 +335,13 @@ int  pfk_pass_check(const pfk_pass *p);
 /* Kernel families with a kernel for the pass shape (bit mask):
  * PFK_HAS_POW2 register kernels for power-of-two lengths 64..4096,
  * PFK_HAS_SMALL one-line-per-lane kernels for short c2c lengths,
- * PFK_HAS_MFMA MFMA kernels (complex64 arithmetic forms).  The general
+ * PFK_HAS_MFMA MFMA kernels (complex64 arithmetic forms), PFK_HAS_MIXED
+ * the mixed-radix kernel.  The general
  * kernel covers every pass.  With PFFT_AMD_GENERIC_ONLY=1 the mask is 0. */
 #define PFK_HAS_POW2  1
 #define PFK_HAS_SMALL 2
 #define PFK_HAS_MFMA  4
+#define PFK_HAS_MIXED 8
 int  pfk_pass_kernels(const pfk_pass *p);
 /* 1 if the pass is plain (every input and output position present, no
  * modulation or weights): the instantiations without masks run it */

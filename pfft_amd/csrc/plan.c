@@ -120,25 +120,70 @@ static int same_geo(const arrgeo *a, const arrgeo *b) {
 }
 
 
+/* Device copy of `count` complex values given in double, or NULL. */
+static const void *upload_table(pa_plan *p, const double *h, INT count) {
+  void *d = NULL;
+  if (p->prec == PFK_F64) {
+    const size_t bytes = sizeof(double) * 2 * (size_t)count;
+    if (pfk_malloc(&d, bytes)) return NULL;
+    p->tw_bufs[p->ntw++] = d;
+    return pfk_memcpy_h2d(d, h, bytes) ? NULL : d;
+  }
+  const size_t bytes = sizeof(float) * 2 * (size_t)count;
+  float *f = (float *)malloc(bytes);
+  if (!f) return NULL;
+  for (INT i = 0; i < 2 * count; i++) f[i] = (float)h[i];
+  const int err = pfk_malloc(&d, bytes) != 0;
+  if (!err) p->tw_bufs[p->ntw++] = d;
+  const int bad = err || pfk_memcpy_h2d(d, f, bytes);
+  free(f);
+  return bad ? NULL : d;
+}
+
 static const void *make_twiddles(pa_plan *p, INT N, INT count, int sign) {
   double *h = (double *)malloc(sizeof(double) * 2 * (size_t)(count > 0 ? count : 1));
   if (!h) return NULL;
   pa_twiddles((long)N, (long)count, sign, h);
-  void *d = NULL;
-  size_t bytes;
-  if (p->prec == PFK_F64) {
-    bytes = sizeof(double) * 2 * (size_t)count;
-    if (pfk_malloc(&d, bytes) || pfk_memcpy_h2d(d, h, bytes)) { free(h); return NULL; }
-  } else {
-    float *f = (float *)malloc(sizeof(float) * 2 * (size_t)count);
-    for (INT i = 0; i < 2 * count; i++) f[i] = (float)h[i];
-    bytes = sizeof(float) * 2 * (size_t)count;
-    if (pfk_malloc(&d, bytes) || pfk_memcpy_h2d(d, f, bytes)) { free(f); free(h); return NULL; }
-    free(f);
-  }
+  const void *d = upload_table(p, h, count);
   free(h);
-  p->tw_bufs[p->ntw++] = d;
   return d;
+}
+
+/* Twiddles of pass `ps` (computed length nf, sign): W_nf^m, m < nf, and behind
+ * them, in the same allocation, the mixed-radix kernel's stage table
+ * (pfk.h), whose entries are powers of W_nf too.  Sets ps->tw and the mixed
+ * fields; nonzero on failure. */
+static int make_pass_twiddles(pa_plan *p, pfk_pass *ps, INT nf, int sign) {
+  ps->mix_n = pfk_mix_factorize(nf, ps->mix_rad);
+  INT extra = 0, L = 1;
+  for (int s = 0; s < ps->mix_n; s++) {
+    if (s) extra += (ps->mix_rad[s] - 1) * L;
+    if (ps->mix_rad[s] > 16) extra += ps->mix_rad[s];
+    L *= ps->mix_rad[s];
+  }
+  double *h = (double *)malloc(sizeof(double) * 2 * (size_t)(nf + extra));
+  if (!h) return 1;
+  pa_twiddles((long)nf, (long)nf, sign, h);
+  double *o = h + 2 * nf;
+  L = 1;
+  for (int s = 0; s < ps->mix_n; s++) {
+    const INT R = ps->mix_rad[s], M = nf / (L * R);
+    for (INT r = 1; s && r < R; r++)
+      for (INT k = 0; k < L; k++, o += 2) {
+        o[0] = h[2 * (r * k * M)];
+        o[1] = sign < 0 ? h[2 * (r * k * M) + 1] : -h[2 * (r * k * M) + 1];
+      }
+    for (INT r = 0; R > 16 && r < R; r++, o += 2) {
+      o[0] = h[2 * (r * (nf / R))];
+      o[1] = sign < 0 ? h[2 * (r * (nf / R)) + 1] : -h[2 * (r * (nf / R)) + 1];
+    }
+    L *= R;
+  }
+  ps->tw = upload_table(p, h, nf + extra);
+  free(h);
+  if (!ps->tw) return 1;
+  ps->twm = (const char *)ps->tw + (size_t)nf * (p->prec == PFK_F64 ? 16 : 8);
+  return 0;
 }
 
 /* Table of a long line nf = n1 * n2 (pfk.h): W_n1^m (m < n1), W_n2^m
@@ -642,7 +687,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
         int64_t l1, l2;
         int path;
         (void)pfk_r2r_inner(ps, &in, &l1, &l2, &path);
-        ps->tw = make_twiddles(p, in.nf, in.nf, in.sign);
+        if (make_pass_twiddles(p, ps, in.nf, in.sign)) goto fail;
         p->tw_adj[k] = ps->tw;   /* r2r plans have no adjoint */
         const int mode = pfk_r2r_mode(kinds[d]);
         if (path == 1 && mode != 2) {
@@ -661,7 +706,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
         ps->tw = make_long_twiddles(p, ps->nf, ps->n1, ps->sign);
         p->tw_adj[k] = make_long_twiddles(p, ps->nf, ps->n1, -ps->sign);
       } else {
-        ps->tw = make_twiddles(p, ps->nf, ps->nf, ps->sign);
+        if (make_pass_twiddles(p, ps, ps->nf, ps->sign)) goto fail;
         p->tw_adj[k] = make_twiddles(p, ps->nf, ps->nf, -ps->sign);
       }
       if (!ps->tw || !p->tw_adj[k]) goto fail;
@@ -1146,7 +1191,7 @@ static const char *kernel_name(const pfk_pass *ps) {
   if (ps->n1) return "long-two-step";
   if (ps->r2r_path) return "r2r-inner-fft";
   const int fam = pfk_pass_kernels(ps);
-  const int lm = (ps->variant & 8) && ps->kind != PFK_R2R &&
+  const int lm = (ps->variant & 8) && ps->variant != 9 && ps->kind != PFK_R2R &&
                  (ps->prec == PFK_F32 || pfk_pass_plain(ps));
   if (fam & PFK_HAS_MFMA) {
     static const char *nm[2][2] = {{"mfma-f32", "mfma-f32-lm"}, {"mfma-bf16x2", "mfma-bf16x2-lm"}};
@@ -1154,6 +1199,7 @@ static const char *kernel_name(const pfk_pass *ps) {
   }
   if (ps->variant == 1) return "general";
   if (ps->variant == 3 && (fam & PFK_HAS_SMALL)) return "small";
+  if (ps->variant == 9 && (fam & PFK_HAS_MIXED)) return "mixed";
   if (fam & PFK_HAS_POW2) {
     static const char *nm[2][4] = {
         {"fast", "fast-narrow", "fast-grid", "fast-narrow-grid"},
@@ -1161,7 +1207,7 @@ static const char *kernel_name(const pfk_pass *ps) {
     return nm[lm][((ps->variant & 3) == 2 ? 1 : 0) + ((ps->variant & 4) ? 2 : 0)];
   }
   if (fam & PFK_HAS_SMALL) return "small";
-  return "general";
+  return (fam & PFK_HAS_MIXED) ? "mixed" : "general";
 }
 
 /* One line per pass: kind, length, strides, batch and tile geometry,
@@ -1181,7 +1227,10 @@ int pa_plan_describe(const pa_plan *p, char *buf, size_t len) {
                           (long long)ps->zout, (long long)ps->sin, (long long)ps->sout,
                           (long long)ps->text, (long long)ps->tsin, (long long)ps->tsout, ps->nb,
                           p->src_role[k], p->dst_role[k], kernel_name(ps),
-                          (ps->xcd_remap && !strncmp(kernel_name(ps), "fast", 4)) ? "+xcd" : "");
+                          (ps->xcd_remap && (!strncmp(kernel_name(ps), "fast", 4) ||
+                                             !strcmp(kernel_name(ps), "mixed")))
+                              ? "+xcd"
+                              : "");
   }
   return 0;
 }

@@ -29,159 +29,11 @@
 // another thread, so both use one extra LDS exchange.
 #pragma once
 #include <stdlib.h>
-#include "pfk_internal.hpp"
+#include "pass_access.hpp"
+#include "dft_regs.hpp"
 #include "pow2_launch.hpp"
 
 namespace pfk {
-
-template <typename T>
-using C2 = cpx<T>;
-
-template <typename T>
-__device__ __forceinline__ C2<T> cadd(C2<T> a, C2<T> b) { return C2<T>{a.x + b.x, a.y + b.y}; }
-template <typename T>
-__device__ __forceinline__ C2<T> csub(C2<T> a, C2<T> b) { return C2<T>{a.x - b.x, a.y - b.y}; }
-// multiply by SIGN*i
-template <int SIGN, typename T>
-__device__ __forceinline__ C2<T> mul_si(C2<T> a) {
-  return SIGN < 0 ? C2<T>{a.y, -a.x} : C2<T>{-a.y, a.x};
-}
-
-template <int SIGN, typename T>
-__device__ __forceinline__ void dft2(C2<T> &a, C2<T> &b) {
-  const C2<T> s = cadd(a, b), d = csub(a, b);
-  a = s;
-  b = d;
-}
-
-// in-place DFT-4 of (a0,a1,a2,a3) with W4 = SIGN*i
-template <int SIGN, typename T>
-__device__ __forceinline__ void dft4(C2<T> &a0, C2<T> &a1, C2<T> &a2, C2<T> &a3) {
-  const C2<T> c0 = cadd(a0, a2), c1 = csub(a0, a2);
-  const C2<T> c2 = cadd(a1, a3), c3 = mul_si<SIGN>(csub(a1, a3));
-  a0 = cadd(c0, c2);
-  a2 = csub(c0, c2);
-  a1 = cadd(c1, c3);
-  a3 = csub(c1, c3);
-}
-
-// in-place DFT-8 of v[0..7] (natural order in and out)
-template <int SIGN, typename T>
-__device__ __forceinline__ void dft8(C2<T> *v) {
-  C2<T> e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
-  C2<T> o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
-  dft4<SIGN>(e0, e1, e2, e3);
-  dft4<SIGN>(o0, o1, o2, o3);
-  const T s = (T)0.70710678118654752440084436210484903928L;
-  // W8^1 = s(1 + SIGN i), W8^2 = SIGN i, W8^3 = s(-1 + SIGN i)
-  const C2<T> t1{s * (o1.x - (SIGN) * o1.y), s * (o1.y + (SIGN) * o1.x)};
-  const C2<T> t2 = mul_si<SIGN>(o2);
-  const C2<T> t3{s * (-o3.x - (SIGN) * o3.y), s * (-o3.y + (SIGN) * o3.x)};
-  v[0] = cadd(e0, o0);
-  v[4] = csub(e0, o0);
-  v[1] = cadd(e1, t1);
-  v[5] = csub(e1, t1);
-  v[2] = cadd(e2, t2);
-  v[6] = csub(e2, t2);
-  v[3] = cadd(e3, t3);
-  v[7] = csub(e3, t3);
-}
-
-// Global accesses.  Streaming (nontemporal) accesses leave nothing behind in
-// the 256 MB memory-side cache, kept ones do: an array that the next pass or
-// the next chunk of the plan touches again while it is still there is kept
-// (pfk_pass.cache), everything else is streamed.  The kernels' KP
-// instantiations choose at run time; the others stream without looking (the
-// choice alone cost passes that stream 1%: 512^3 complex128 pair 2.29 -> 2.31
-// ms).
-template <typename T>
-__device__ __forceinline__ C2<T> ld_stream(const C2<T> *p) {
-  typedef T v2 __attribute__((ext_vector_type(2)));
-  const v2 v = __builtin_nontemporal_load(reinterpret_cast<const v2 *>(p));
-  return C2<T>{v.x, v.y};
-}
-template <typename T>
-__device__ __forceinline__ void st_stream(C2<T> *p, C2<T> v) {
-  typedef T v2 __attribute__((ext_vector_type(2)));
-  v2 w;
-  w.x = v.x;
-  w.y = v.y;
-  __builtin_nontemporal_store(w, reinterpret_cast<v2 *>(p));
-}
-// loads v[m] = *at(m), m < N, kept or streamed: one uniform branch around the
-// whole batch of loads
-template <bool KP, int N, typename T, typename At>
-__device__ __forceinline__ void ld_batch(const pfk_pass &P, C2<T> *v, At at) {
-  if (KP && (P.cache & PFK_KEEP_SRC)) {
-#pragma unroll
-    for (int m = 0; m < N; ++m) v[m] = *at(m);
-  } else {
-#pragma unroll
-    for (int m = 0; m < N; ++m) v[m] = ld_stream(at(m));
-  }
-}
-template <typename T>
-__device__ __forceinline__ void st_elem(const bool keep, C2<T> *p, C2<T> v) {
-  if (keep) *p = v;
-  else st_stream(p, v);
-}
-// stores *at(m) = v[m], m < N
-template <int N, typename T, typename At>
-__device__ __forceinline__ void st_batch(const bool keep, const C2<T> *v, At at) {
-  if (keep) {
-#pragma unroll
-    for (int m = 0; m < N; ++m) *at(m) = v[m];
-  } else {
-#pragma unroll
-    for (int m = 0; m < N; ++m) st_stream(at(m), v[m]);
-  }
-}
-
-// in-place DFT-16 of v[0..15] as 4x4: DFT-4 over stride-4 groups, twiddle
-// W16^(r*q), DFT-4 across groups
-template <int SIGN, typename T>
-__device__ __forceinline__ void dft16(C2<T> *v) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) dft4<SIGN>(v[r], v[r + 4], v[r + 8], v[r + 12]);
-  // v[r + 4q] now holds sub-DFT output q of group r; multiply by W16^(r*q)
-  const T c1 = (T)0.92387953251128675612818318939678828682L;  // cos(pi/8)
-  const T s1 = (T)0.38268343236508977172845998403039886676L;  // sin(pi/8)
-  const T h = (T)0.70710678118654752440084436210484903928L;
-  const T S = (T)SIGN;
-  // W16^1 = c1 + S i s1, W16^2 = h + S i h, W16^3 = s1 + S i c1,
-  // W16^4 = S i, W16^6 = -h + S i h, W16^9 = -c1 - S i s1
-  const C2<T> w1{c1, S * s1}, w2{h, S * h}, w3{s1, S * c1};
-  const C2<T> w6{-h, S * h}, w9{-c1, -S * s1};
-  v[5] = cmul(v[5], w1);
-  v[9] = cmul(v[9], w2);
-  v[13] = cmul(v[13], w3);
-  v[6] = cmul(v[6], w2);
-  v[10] = mul_si<SIGN>(v[10]);
-  v[14] = cmul(v[14], w6);
-  v[7] = cmul(v[7], w3);
-  v[11] = cmul(v[11], w6);
-  v[15] = cmul(v[15], w9);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) dft4<SIGN>(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-  // output k = q + 4*s sits in v[4q + s]: transpose the 4x4 index
-  C2<T> o[16];
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int t = 0; t < 4; ++t) o[q + 4 * t] = v[4 * q + t];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = o[k];
-}
-
-// +-1 modulation factor of index j, computed with selects only: a branch
-// here would sit between a load and its use and make the compiler wait for
-// every load before issuing the next one.
-template <typename T>
-__device__ __forceinline__ T msign(const pfk_mod &m, int64_t j) {
-  const int64_t t = j + m.start;
-  const int s = (m.on && t < m.half) ? ((t & 1) ? -m.extra : m.extra) : 1;
-  return (T)s;
-}
 
 constexpr int ilog2c(int n) { return n <= 1 ? 0 : 1 + ilog2c(n / 2); }
 
@@ -351,63 +203,6 @@ __device__ __forceinline__ void fft_stages_sw(C2<T> *v, int *pos, C2<T> *lds, co
   } else if constexpr (REM > 1) {
     stage<T, NF, E, REM, L, SIGN, true>(v, pos, t, tw);
   }
-}
-
-struct TileCtx {
-  int64_t sb, db;
-  int64_t c0;   // first line of the tile along the tile dimension
-  int nl;
-};
-
-// Workgroups are dispatched round-robin over the 8 XCDs (each with its own
-// L2).  With remap on, XCD x runs a contiguous range of tiles in order, so
-// tiles that share cache lines at their edges run on the same L2 close in
-// time.  The map is a bijection on [0, n) for any n; item i runs on XCD
-// i mod 8 because the persistent grid is a multiple of 8.
-__device__ __forceinline__ int64_t xcd_remap(int64_t b, int64_t n) {
-  const int64_t q = n >> 3, r = n & 7;
-  const int64_t x = b & 7, j = b >> 3;
-  return x * q + (x < r ? x : r) + j;
-}
-
-// Tile of work item `item` (0 <= item < ntiles).  Tile counts below 2^32
-// (every practical pass) decode with 32-bit divisions, several times
-// shorter than the 64-bit chain.
-__device__ __forceinline__ TileCtx tile_at(const pfk_pass &P, int C, int64_t item,
-                                           int64_t ntiles) {
-  const int64_t ntt = (P.text + C - 1) / C;
-  const int64_t tileid = P.xcd_remap ? xcd_remap(item, ntiles) : item;
-  int64_t tt, sb = 0, db = 0;
-  if (ntiles <= (int64_t)0xFFFFFFFFu) {
-    uint32_t id = (uint32_t)tileid;
-    const uint32_t n32 = (uint32_t)ntt;
-    tt = id % n32;
-    id /= n32;
-    for (int i = 0; i < P.nb; ++i) {
-      const uint32_t e = (uint32_t)P.bext[i];
-      const uint32_t d = id % e;
-      id /= e;
-      sb += (int64_t)d * P.bsin[i];
-      db += (int64_t)d * P.bsout[i];
-    }
-  } else {
-    tt = tileid % ntt;
-    int64_t bflat = tileid / ntt;
-    for (int i = 0; i < P.nb; ++i) {
-      const int64_t e = P.bext[i];
-      const int64_t d = bflat % e;
-      bflat /= e;
-      sb += d * P.bsin[i];
-      db += d * P.bsout[i];
-    }
-  }
-  const int64_t c0 = tt * C;
-  TileCtx r;
-  r.c0 = c0;
-  r.nl = (int)((P.text - c0) < C ? (P.text - c0) : C);
-  r.sb = sb + c0 * P.tsin;
-  r.db = db + c0 * P.tsout;
-  return r;
 }
 
 // Persistent pass kernels.  A fixed grid of resident workgroups walks the

@@ -20,7 +20,9 @@
  *   (8,r) (12,r) as (0,r) (4,r) with line-major lane order (complex64
  *         passes whose lines are contiguous on at least one side);
  *   (3,0) short-length kernel, one line per lane;
- *   (1,0) the general kernel.
+ *   (9,0) (9,1) the mixed-radix kernel, where the power-of-two kernels do not
+ *         reach or the tile dimension fills less than one of their tiles;
+ *   (1,0) the general kernel, where the mixed-radix one is no candidate.
  * A pass with one candidate is not timed.  All candidates compute the
  * same transform (the power-of-two variants bit-identically, the others
  * with their own factorisations).  A pass run by an MFMA kernel keeps it
@@ -128,7 +130,7 @@ int pa_wisdom_import(const char *filename) {
     int v, r;
     double ms;
     if (!fgets(line, sizeof line, f) || sscanf(line, "%319s %d %d %lf", key, &v, &r, &ms) != 4 ||
-        v < 0 || v > 14 || ((v & 1) && v != 1 && v != 3) || r < 0 || r > 1) {
+        v < 0 || v > 14 || ((v & 1) && v != 1 && v != 3 && v != 9) || r < 0 || r > 1) {
       ok = 0;
       break;
     }
@@ -216,8 +218,9 @@ int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort) {
   const char *rv = getenv("PFFT_AMD_XCD_REMAP");
   const int remap_fixed = (rv && *rv) ? (rv[0] == '1') : -1;
   const int reps = (effort & PFFT_EXHAUSTIVE) ? 10 : (effort & PFFT_PATIENT) ? 6 : 3;
-  static const int cand[14][2] = {{0, 0}, {0, 1}, {2, 0},  {2, 1},  {4, 0},  {4, 1},  {6, 0},
-                                  {6, 1}, {8, 0}, {8, 1}, {12, 0}, {12, 1}, {3, 0}, {1, 0}};
+  static const int cand[16][2] = {{0, 0}, {0, 1}, {2, 0},  {2, 1},  {4, 0},  {4, 1},  {6, 0},
+                                  {6, 1}, {8, 0}, {8, 1}, {12, 0}, {12, 1}, {3, 0}, {9, 0},
+                                  {9, 1}, {1, 0}};
   /* line-major lane order: c2c passes whose lines are contiguous on one
    * side and contiguous or adjacent along the tile on the other (the
    * kernels switch lane order at an LDS exchange), and real passes whose
@@ -228,6 +231,7 @@ int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort) {
       (ps->kind == PFK_R2C && ps->sout == 1) || (ps->kind == PFK_C2R && ps->sin == 1);
   const int lm_ok = lm_shape && (ps->prec == PFK_F32 || pfk_pass_plain(ps));
   const int fam = pfk_pass_kernels(ps);
+  const int mixed = (fam & PFK_HAS_MIXED) && (!(fam & PFK_HAS_POW2) || ps->text < 8);
   void *e0 = NULL, *e1 = NULL;
   if (pfk_event_create(&e0) || pfk_event_create(&e1)) {
     if (e0) pfk_event_destroy(e0);
@@ -236,15 +240,16 @@ int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort) {
   const int v0 = ps->variant, r0 = ps->xcd_remap;
   int best_v = v0, best_r = r0, err = 0;
   double best = -1;
-  for (int c = 0; c < 14 && !err; c++) {
+  for (int c = 0; c < 16 && !err; c++) {
     const int v = cand[c][0], r = cand[c][1];
-    const int pow2 = v != 1 && v != 3;
-    if ((v & 8) && !lm_ok) continue;
+    const int pow2 = v != 1 && v != 3 && v != 9;
+    if (pow2 && (v & 8) && !lm_ok) continue;
     if (fam & PFK_HAS_MFMA) {   /* the user's arithmetic form: grid, lane order, XCD order vary */
       if ((v & 3) || (remap_fixed >= 0 && r != remap_fixed)) continue;
     } else if (pow2 && !(fam & PFK_HAS_POW2)) continue;
     if (v == 3 && !(fam & PFK_HAS_SMALL)) continue;
-    if (pow2 && remap_fixed >= 0 && r != remap_fixed) continue;
+    if (v == 9 ? !mixed : v == 1 && mixed) continue;
+    if ((pow2 || v == 9) && remap_fixed >= 0 && r != remap_fixed) continue;
     ps->variant = v;
     ps->xcd_remap = r;
     const double t = time_launches(ps, src, dst, reps, e0, e1);
