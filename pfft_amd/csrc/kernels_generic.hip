@@ -39,7 +39,9 @@ __global__ void __launch_bounds__(256)
 k_pass_generic(const pfk_pass P, const int C, const int pitch, const int64_t tile_base,
                const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
+  stamp_begin(P);
   pass_tile<T, KIND, EPT>(P, C, pitch, tile_base + blockIdx.x, src, dst, smem_raw);
+  stamp_end(P);
 }
 
 // number of complex LDS slots one line needs
@@ -726,6 +728,8 @@ using namespace pfk;
 
 extern "C" {
 
+static void stamps_init(void);
+
 int pfk_init(void) {
   if (g_stream) return 0;
   hipError_t e = hipFree(0);
@@ -740,6 +744,7 @@ int pfk_init(void) {
   g_generic_only = (go && go[0] == '1') ? 1 : 0;
   e = hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking);
   if (e != hipSuccess) { set_error("pfk_init(hipStreamCreate)", e); g_stream = nullptr; return 1; }
+  stamps_init();
   return 0;
 }
 
@@ -907,6 +912,38 @@ int pfk_launch_pass(const pfk_pass *p, const void *src, void *dst) {
   if (r == 0) return 0;
   if (r < 0) return 1;
   return launch_generic(p, src, dst);
+}
+
+int pfk_pass_stamps(const pfk_pass *p) {
+  return !p->n1 && !(p->kind == PFK_R2R && p->r2r_path) && !p->mfma;
+}
+
+#define STAMP_BLOCKS 64
+static uint64_t *g_stamps;           // STAMP_BLOCKS * PFK_STAMPS words, pinned
+static double g_stamp_period;        // seconds per tick
+static void stamps_init(void) {      // from pfk_init, once
+  int dev = 0, khz = 0;
+  (void)hipGetDevice(&dev);
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess ||
+      khz <= 0 ||
+      hipHostMalloc((void **)&g_stamps, STAMP_BLOCKS * PFK_STAMPS * sizeof(uint64_t),
+                    hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    g_stamps = nullptr;
+    return;
+  }
+  g_stamp_period = 1e-3 / khz;
+}
+uint64_t *pfk_stamps(void) {
+  static unsigned next = 0;
+  if (pfk_init() || !g_stamps) return nullptr;
+  uint64_t *s = g_stamps + (__atomic_fetch_add(&next, 1u, __ATOMIC_RELAXED) % STAMP_BLOCKS) *
+                               PFK_STAMPS;
+  memset(s, 0, PFK_STAMPS * sizeof(uint64_t));
+  return s;
+}
+double pfk_stamp_seconds(uint64_t a, uint64_t b) {
+  return b > a ? (double)(b - a) * g_stamp_period : 0.0;
 }
 
 int pfk_event_create(void **ev) {

@@ -13,7 +13,9 @@ __global__ void __launch_bounds__(256)
 k_small(const pfk_pass P, const int64_t tile_base, const T *__restrict__ src,
         T *__restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
+  stamp_begin(P);
   small_tile<T, NF>(P, tile_base + blockIdx.x, src, dst, smem_raw);
+  stamp_end(P);
 }
 
 template <typename T, int NF, int KIND>
@@ -21,7 +23,9 @@ __global__ void __launch_bounds__(256)
 k_small_real(const pfk_pass P, const int64_t tile_base, const T *__restrict__ src,
              T *__restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
+  stamp_begin(P);
   small_split_real_tile<T, NF, KIND>(P, tile_base + blockIdx.x, src, dst, smem_raw);
+  stamp_end(P);
 }
 
 // The length rule of small_covers for even r2c / c2r passes (without the

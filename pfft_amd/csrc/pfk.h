@@ -138,6 +138,10 @@ typedef struct pfk_pass {
   int32_t mix_n;
   int32_t mix_rad[PFK_MIX_MAXST];
   const void *twm;
+  /* times of the pass (pfk_stamps; NULL: none): its first workgroup stores
+   * the clock to `stamp` when it starts, the last PFK_STAMP_ENDS workgroups
+   * store it to stamp_end[...] when they end */
+  uint64_t *stamp, *stamp_end;
   /* element counts of the src/dst buffers, for host-side bounds checks */
   int64_t src_elems, dst_elems;
 } pfk_pass;
@@ -147,6 +151,8 @@ typedef struct pfk_pass {
  * of streaming ones.  Kernels without streaming accesses ignore it. */
 #define PFK_KEEP_SRC 1
 #define PFK_KEEP_DST 2
+
+#define PFK_STAMP_ENDS 32
 
 /* Longest computed line one workgroup transforms. */
 #define PFK_MAXLINE 4096
@@ -352,6 +358,20 @@ int  pfk_event_create(void **ev);
 int  pfk_event_record(void *ev);
 int  pfk_event_elapsed_ms(void *ev0, void *ev1, float *ms);
 int  pfk_event_destroy(void *ev);
+
+/* Stamps of one execution: PFK_STAMPS words of pinned host memory, zeroed, for
+ * start times (pfk_pass.stamp) and, from word PFK_STAMPS - PFK_STAMP_ENDS on,
+ * the end of the last pass.  The blocks are a fixed ring that executions
+ * take in turn; one that overlaps with 63 others may find its times
+ * overwritten (times only).  NULL if there is no memory.
+ * Why not events: an event between two passes keeps the second from starting
+ * for 5.7 us (none between launches without one). */
+#define PFK_STAMPS 48
+uint64_t *pfk_stamps(void);
+double pfk_stamp_seconds(uint64_t from, uint64_t to);
+/* 1 if the kernels that run the pass write its stamps (single launch, not the
+ * MFMA forms) */
+int  pfk_pass_stamps(const pfk_pass *p);
 
 /* Complex conjugation / scaling utility kernels on device arrays. */
 int  pfk_scale(void *data, int prec, int64_t nreal, double factor);

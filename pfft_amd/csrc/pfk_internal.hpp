@@ -25,6 +25,19 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Times of a pass (pfk_pass.stamp): at its start from workgroup 0, at its end
+// from the last workgroups of the grid, dispatched last and ending about last.
+// Every lane stores: a test of the thread index would keep it in a register to
+// the end, one more than the 128 that leave the 512-point complex128 kernels
+// 16 waves per CU (512^3 pair 2.28 -> 2.38 ms).
+__device__ __forceinline__ void stamp_begin(const pfk_pass &P) {
+  if (P.stamp && blockIdx.x == 0) *P.stamp = wall_clock64();
+}
+__device__ __forceinline__ void stamp_end(const pfk_pass &P) {
+  const unsigned k = gridDim.x - 1 - blockIdx.x;
+  if (P.stamp_end && k < PFK_STAMP_ENDS) P.stamp_end[k] = wall_clock64();
+}
+
 extern hipStream_t g_stream;
 extern int g_generic_only;   // PFFT_AMD_GENERIC_ONLY=1: route every pass to the general kernel
 extern int g_max_lds;

@@ -71,7 +71,8 @@ struct pa_plan {
   void *work2[PA_MAXRNK];        /* long real-line passes: the same again */
   void *r2rw[2];                 /* r2r passes on the inner real FFT: its input / output */
   /* execution timer (kernel/timer.c fields): pass k adds its device time
-   * to trafo[tslot[k]]; events tev[0..npass] bracket the passes */
+   * to trafo[tslot[k]]; events tev[0..npass] bracket the passes, or, where
+   * every pass writes stamps, tev[0] is NULL */
   pa_timer *timer;
   int tslot[PA_MAXRNK];
   void *tev[PA_MAXRNK + 1];
@@ -819,7 +820,11 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
     const int d = ord[k];
     p->tslot[k] = first0 ? (d >= r ? 2 * r + 1 : r + 1 + d) : (d >= r ? 0 : r - d);
   }
-  for (int k = 0; k <= R; k++)
+  /* pass times: stamps written by the kernels, or events where a pass has
+   * none (or the stamps no memory) */
+  int stamped = R < PFK_STAMPS - PFK_STAMP_ENDS && pfk_stamps() != NULL;
+  for (int k = 0; k < R; k++) stamped &= pfk_pass_stamps(&p->pass[k]);
+  for (int k = 0; k <= R && !stamped; k++)
     if (pfk_event_create(&p->tev[k])) {
       pa_error("event creation failed: %s", pfk_last_error());
       goto fail;
@@ -848,6 +853,7 @@ void *pa_plan_out(const pa_plan *p) { return p->out; }
 static void run(const pa_plan *p, void *in, void *out, int adjoint) {
   if (!p) return;
   const double t0 = wall_seconds();
+  uint64_t *const stamps = p->tev[0] ? NULL : pfk_stamps();   /* else events */
   if (adjoint && p->is_r2r) {
     pa_error("the adjoint pipeline is not available for r2r plans");
     return;
@@ -883,14 +889,16 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
     }
   }
   void *bufs[4] = {din, dout, p->scratch[0], p->scratch[1]};
-  int err = pfk_event_record(p->tev[0]);
+  int err = p->tev[0] ? pfk_event_record(p->tev[0]) : 0;
   for (int i = 0; i < p->npass && !err; i++) {
     const int k = adjoint ? p->npass - 1 - i : i;
     const pfk_pass *fw = &p->pass[k];
+    pfk_pass a = *fw;
+    a.stamp = stamps ? stamps + i : NULL;
+    a.stamp_end = stamps && i == p->npass - 1 ? stamps + PFK_STAMPS - PFK_STAMP_ENDS : NULL;
     if (!adjoint) {
-      err = pfk_launch_pass(fw, bufs[p->src_role[k]], bufs[p->dst_role[k]]);
+      err = pfk_launch_pass(&a, bufs[p->src_role[k]], bufs[p->dst_role[k]]);
     } else {
-      pfk_pass a = *fw;
       a.sign = -fw->sign;
       a.nin = fw->nout; a.zin = fw->zout;
       a.nout = fw->nin; a.zout = fw->zin;
@@ -908,11 +916,20 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
       static const int swap_io[4] = {ROLE_OUT, ROLE_IN, ROLE_S0, ROLE_S1};
       err = pfk_launch_pass(&a, bufs[swap_io[p->dst_role[k]]], bufs[swap_io[p->src_role[k]]]);
     }
-    if (!err) err = pfk_event_record(p->tev[i + 1]);
+    if (!err && p->tev[0]) err = pfk_event_record(p->tev[i + 1]);
     if (err) pa_error("pass %d launch failed: %s", k, pfk_last_error());
   }
   if (!err && pfk_sync()) { pa_error("execution failed: %s", pfk_last_error()); err = 1; }
-  if (!err) {
+  if (!err && stamps) {
+    uint64_t end = 0;
+    for (int i = PFK_STAMPS - PFK_STAMP_ENDS; i < PFK_STAMPS; i++)
+      if (stamps[i] > end) end = stamps[i];
+    for (int i = 0; i < p->npass; i++) {
+      const int k = adjoint ? p->npass - 1 - i : i;
+      p->timer->trafo[p->tslot[k]] +=
+          pfk_stamp_seconds(stamps[i], i + 1 < p->npass ? stamps[i + 1] : end);
+    }
+  } else if (!err && p->tev[0]) {
     for (int i = 0; i < p->npass; i++) {
       float ms = 0;
       const int k = adjoint ? p->npass - 1 - i : i;

@@ -333,6 +333,7 @@ template <typename T, int NF, int C, int E, int SIGN, bool LM = false, bool TW =
 __global__ void __launch_bounds__(C *NF / E)
 k_c2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const int64_t ntiles,
            const T *__restrict__ src, T *__restrict__ dst) {
+  stamp_begin(P);
   constexpr int TT = NF / E;
   constexpr bool TWL = tw_in_lds<T>(lds_slots<NF, C, LM>(), NF, 0);
   __shared__ C2<T> lds[lds_slots<NF, C, LM>()];
@@ -437,6 +438,7 @@ k_c2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const 
   if constexpr (TWL) lds_barrier();
   while (step(va, vb) && step(vb, va)) {
   }
+  stamp_end(P);
 }
 
 // ------------------------------------------------------------------ r2c
@@ -459,6 +461,7 @@ template <typename T, int NF, int C, int E, int SIGN, bool PL = false, bool LM =
 __global__ void __launch_bounds__(C *NF / E)
 k_r2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const int64_t ntiles,
            const T *__restrict__ src, T *__restrict__ dst) {
+  stamp_begin(P);
   constexpr int TT = NF / E;
   constexpr int H = NF;  // h = n/2
   constexpr bool TWL = tw_in_lds<T>(lds_slots<NF, C, LM>(), NF, NF);
@@ -553,6 +556,7 @@ k_r2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const 
   if constexpr (TWL) lds_barrier();
   while (step(va, vb) && step(vb, va)) {
   }
+  stamp_end(P);
 }
 
 // ------------------------------------------------------------------ c2r
@@ -587,6 +591,7 @@ template <typename T, int NF, int C, int E, int SIGN, bool PL = false, bool LM =
 __global__ void __launch_bounds__(C *NF / E)
 k_c2r_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const int64_t ntiles,
            const T *__restrict__ src, T *__restrict__ dst) {
+  stamp_begin(P);
   constexpr int TT = NF / E;
   constexpr int H = NF;
   constexpr int SLOTS = LM ? lds_slots<NF, C, true>() : (NF + 1) * C;   // with the Nyquist bin
@@ -683,6 +688,7 @@ k_c2r_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const 
   if constexpr (TWL) lds_barrier();
   while (step(va, ha, vb, hb) && step(vb, hb, va, ha)) {
   }
+  stamp_end(P);
 }
 
 // ------------------------------------------------------------------ dispatch
