@@ -893,7 +893,10 @@ int pfk_pass_check(const pfk_pass *p) {
 
 int pfk_launch_pass(const pfk_pass *p, const void *src, void *dst) {
   if (pfk_init()) return 1;
-  if (p->kind == PFK_R2R && p->r2r_path) return r2r_real_path(p, src, dst);
+  if (p->kind == PFK_R2R && p->r2r_path) {
+    const int f = g_generic_only ? 1 : launch_mixed(p, src, dst);
+    return f > 0 ? r2r_real_path(p, src, dst) : f < 0;
+  }
   if (p->n1) return launch_long(p, src, dst);
   if (!g_generic_only && p->mfma) {
     const int m = launch_mfma(p, src, dst);
@@ -915,7 +918,8 @@ int pfk_launch_pass(const pfk_pass *p, const void *src, void *dst) {
 }
 
 int pfk_pass_stamps(const pfk_pass *p) {
-  return !p->n1 && !(p->kind == PFK_R2R && p->r2r_path) && !p->mfma;
+  if (p->kind == PFK_R2R && p->r2r_path) return !g_generic_only && mixed_covers(p);
+  return !p->n1 && !p->mfma;
 }
 
 #define STAMP_BLOCKS 64

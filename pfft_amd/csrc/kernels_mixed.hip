@@ -8,6 +8,10 @@ int launch_mixed_f64(const pfk_pass *p, const MixGeo &g, int nt, size_t lds, con
                      void *dst);
 int launch_mixed_f32(const pfk_pass *p, const MixGeo &g, int nt, size_t lds, const void *src,
                      void *dst);
+int launch_mixed_r2r_f64(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
+                         const void *src, void *dst);
+int launch_mixed_r2r_f32(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
+                         const void *src, void *dst);
 
 static uint32_t recip(int64_t d) {   // div_m
   return d <= 1 ? 0 : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
@@ -29,7 +33,11 @@ static bool even_strides(const pfk_pass *p, bool in) {
 static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *dst) {
   const bool f64 = p->prec == PFK_F64;
   const size_t esz = f64 ? 16 : 8;
-  const int nf = (int)p->nf;
+  const bool r2r = p->kind == PFK_R2R;
+  const int nf = !r2r ? (int)p->nf
+                 : pfk_r2r_mode(p->r2r) == 0 ? (int)(pfk_r2r_inner_len(p->r2r, p->n) / 2)
+                                             : (int)(p->n / 2);
+  g->m = nf;
   int L = 1, off = 0;
   g->nst = p->mix_n;
   g->big = 0;
@@ -51,7 +59,8 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
     L *= R;
   }
   const bool real = p->kind != PFK_C2C, even = !(p->n & 1);
-  const int rows = (p->kind == PFK_C2R && even) ? nf + 1 : nf;
+  int rows = (p->kind == PFK_C2R && even) ? nf + 1 : nf;   // complex slots of a line
+  if (r2r && pfk_r2r_mode(p->r2r) == 1) rows = nf + 1;   // r2r_put
   const size_t ua = 2 * (f64 ? sizeof(double) : sizeof(float));
   g->lm_ld = p->sin == 1;
   g->lm_st = p->sout == 1;
@@ -65,8 +74,8 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
     g->vec = p->sout == 1 && p->nout == p->n && !p->zout && !p->omod.on &&
              even_strides(p, false) && (uintptr_t)dst % ua == 0;
   g->ntw = off;
-  g->mload = recip(rows);
-  g->mstore = recip(p->nout);
+  g->mload = recip(r2r ? p->n : rows);
+  g->mstore = recip(r2r && pfk_r2r_mode(p->r2r) == 0 ? nf + 1 : p->nout);
   g->mrow = recip(nf);
   g->keep_ld = (p->cache & PFK_KEEP_SRC) != 0;
   g->keep_st = (p->cache & PFK_KEEP_DST) != 0;
@@ -82,9 +91,10 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
   int64_t lines = p->text;
   for (int i = 0; i < p->nb; i++) lines *= p->bext[i];
   const int cmin = g->big ? 8 : 1;
-  const int cseg = (g->lm_ld && g->lm_st) ? (g->big ? 8 : 2) : (int)(128 / esz);
+  const int seg = (int)(128 / esz) * (r2r ? 2 : 1);   // lines of a 128-byte segment
+  const int cseg = (g->lm_ld && g->lm_st) ? (g->big ? 8 : 2) : seg;
   const size_t tile = real || !f64 || !(g->lm_ld && g->lm_st) ? 16384 : 32768;
-  int C = (g->lm_ld && g->lm_st) ? 1 : (int)(128 / esz);
+  int C = (g->lm_ld && g->lm_st) ? 1 : seg;
   while (C < 64 && (size_t)(2 * C) * rows * esz <= tile) C *= 2;
   if (C < cmin) C = cmin;
   while (C > cseg && lines < 512 * (int64_t)C) C /= 2;
@@ -110,9 +120,17 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
     }
     nt = (nt + 63) / 64 * 64;
     const size_t lds = mix_lds(g, esz);
+    // r2r: threads beyond the butterflies for the steps before and after the
+    // transform, up to 16 waves a CU at the tile's LDS
+    const int nt16 = 64 * (int)((16 * lds + 160 * 1024 - 1) / (160 * 1024));
+    if (r2r && nt < nt16 && nt16 <= 512) nt = nt16;
     // rows of tiles where rounding them up wastes at most 1/10
     const int64_t up = (p->text + C - 1) / C * C;
     g->text = (up - p->text) * 10 <= p->text ? up : p->text;
+    // r2r lines too long for half a segment, or with matrix-core stages, keep the
+    // three launches
+    if (r2r && g->big) return 0;
+    if (r2r && !(g->lm_ld && g->lm_st) && C < seg / 2) return 0;
     if ((nt <= 512 && lds <= 80 * 1024) || (C == cmin && nt <= 512 && lds <= 158 * 1024))
       return nt;
     if (C == cmin) return 0;
@@ -121,7 +139,11 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
 
 int mixed_covers(const pfk_pass *p) {
   if (!p->twm || p->mix_n < 1 || p->n1 || p->dec_in || p->dec_out || p->twn) return 0;
-  if (p->kind != PFK_C2C && p->kind != PFK_R2C && p->kind != PFK_C2R) return 0;
+  if (p->kind == PFK_R2R) {
+    if (p->r2r_path != 1) return 0;
+  } else if (p->kind != PFK_C2C && p->kind != PFK_R2C && p->kind != PFK_C2R) {
+    return 0;
+  }
   if (p->kind == PFK_C2C && p->hw) return 0;
   MixGeo g;
   return mixed_geo(p, &g, nullptr, nullptr) > 0;
@@ -131,6 +153,9 @@ int launch_mixed(const pfk_pass *p, const void *src, void *dst) {
   if (!mixed_covers(p)) return 1;
   MixGeo g;
   const int nt = mixed_geo(p, &g, src, dst);
+  if (p->kind == PFK_R2R)
+    return p->prec == PFK_F64 ? launch_mixed_r2r_f64(p, g, nt, mix_lds(&g, 16), src, dst)
+                              : launch_mixed_r2r_f32(p, g, nt, mix_lds(&g, 8), src, dst);
   return p->prec == PFK_F64 ? launch_mixed_f64(p, g, nt, mix_lds(&g, 16), src, dst)
                             : launch_mixed_f32(p, g, nt, mix_lds(&g, 8), src, dst);
 }

@@ -59,7 +59,7 @@ static int launch_mixed_k(const pfk_pass *p, const MixGeo &g, int nt, size_t lds
 }
 
 template <typename T>
-static int launch_mixed_t(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
+[[maybe_unused]] static int launch_mixed_t(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
                           const void *src, void *dst) {
   switch (p->kind) {
     case PFK_C2C:
@@ -72,6 +72,26 @@ static int launch_mixed_t(const pfk_pass *p, const MixGeo &g, int nt, size_t lds
       return g.big ? launch_mixed_k<T, PFK_C2R, true>(p, g, nt, lds, src, dst)
                    : launch_mixed_k<T, PFK_C2R, false>(p, g, nt, lds, src, dst);
   }
+}
+
+template <typename T>
+[[maybe_unused]] static int launch_mixed_r2r_t(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
+                              const void *src, void *dst) {
+#define PFK_CASE(K) \
+  case K: return launch_mixed_k<T, mix_kind_r2r(K), false>(p, g, nt, lds, src, dst)
+  switch (p->r2r) {
+    PFK_CASE(PFK_DHT);
+    PFK_CASE(PFK_REDFT00);
+    PFK_CASE(PFK_REDFT01);
+    PFK_CASE(PFK_REDFT10);
+    PFK_CASE(PFK_REDFT11);
+    PFK_CASE(PFK_RODFT00);
+    PFK_CASE(PFK_RODFT01);
+    PFK_CASE(PFK_RODFT10);
+    PFK_CASE(PFK_RODFT11);
+    default: return 1;
+  }
+#undef PFK_CASE
 }
 
 }  // namespace pfk

@@ -26,6 +26,12 @@
 // two dense real products over r for all lines and both components: matrix
 // core work (16x16x4 tiles: 16 outputs q by 8 lines x {re, im} by 4 r).
 //
+// r2r lines of an even inner length (pfk_r2r_inner, path 1) are one launch too:
+// the real line is staged in LDS through the kind's permutation (r2r_put), and
+// its twiddles and combine (r2r_spectrum, r2r_post) run there.  As launches of
+// their own those steps were two further sweeps: 256^3 complex128 DCT-II and
+// DCT-III 1218 -> 578 us, 87-96 us a pass.
+//
 // Bound: the HBM sweep, at 3.7-5.1 TB/s (0.7-1.5 for the general kernel, whose
 // stages sum each output over its radix with a division per element).
 // Forward+backward pairs, general kernel -> this one: c2c 360x300x250
@@ -46,6 +52,7 @@ struct MixGeo {
   int lm_ld, lm_st;        // lanes along the lines on the load / store side
   int vec;                 // real side readable as aligned complex pairs
   int ntw;                 // entries of the stage table
+  int m;                   // computed length (P.nf; r2r: the inner one)
   int big;                 // 1: some stage runs on the matrix cores (a second tile in LDS)
   int keep_ld, keep_st;    // ordinary instead of streaming accesses
   int64_t text;            // tile extent the lines are numbered by (mix_lines)
@@ -55,6 +62,13 @@ struct MixGeo {
   uint32_t mload, mstore;  // reciprocals of the staged load / store loop lengths
   uint32_t mpair[PFK_MIX_MAXST], mrow;   // ... of the pair-sum loop, of nf
 };
+
+// KIND of a kernel: PFK_C2C, PFK_R2C, PFK_C2R, or one of the r2r kinds (a kernel
+// each: with a switch inside, what the kinds have in common is hoisted above it
+// and spilled)
+constexpr int mix_kind_r2r(int r2r) { return 16 + r2r; }
+constexpr bool mix_r2r(int kind) { return kind >= 16; }
+constexpr int mix_r2r_kind(int kind) { return kind - 16; }
 
 // i / d for i * d < 2^32 with m = ceil(2^32 / d) (m = 0: d = 1)
 __device__ __forceinline__ int div_m(int i, uint32_t m) {
@@ -71,6 +85,7 @@ struct MixCtx {
   T *dst;
   const C2<T> *tw;           // LDS: stage table
   C2<T> *lds, *lds2;         // the tile, the second one (G.big)
+  int tid;                   // thread index
   T cj;   // -1 conjugates the input and the output of the forward transform
 };
 
@@ -166,14 +181,184 @@ __device__ __forceinline__ C2<T> c2r_pack(const MixCtx<T> &X, const int c, const
   return z;
 }
 
+// ---- r2r steps around the inner transform (modes in pfk.h) ----
+constexpr int r2r_mode_of(int kind) {   // pfk_r2r_mode
+  return kind == PFK_REDFT01 || kind == PFK_RODFT01   ? 1
+         : kind == PFK_REDFT11 || kind == PFK_RODFT11 ? 2
+                                                      : 0;
+}
+// Element j of the real line (length n) into its row: where the inner complex
+// line of length M (z_q at reals 2q, 2q+1) takes it.
+//   mode 0: the reals v_m whose real FFT the kind needs, z_q = (v_2q, v_2q+1);
+//   mode 1: (x'_q, x'_(n-q)) at q <= M, x'_n = 0 (r2r_spectrum makes z of it);
+//   mode 2: (x'_2q, x'_(n-1-2q)), twiddled when read (mix_staged).
+// x' is x, reversed for the RO kinds of modes 1 and 2.
+template <int KD, typename T>
+__device__ __forceinline__ void r2r_put(T *row, const int n, const int M, const int j,
+                                        const T v) {
+  if constexpr (KD == PFK_DHT) {
+    row[j] = v;
+  } else if constexpr (KD == PFK_REDFT10 || KD == PFK_RODFT10) {
+    // Makhoul: v_m = x_2m, v_(n-1-m') = x_(2m'+1); DST-II: x_j (-1)^j
+    row[(j & 1) ? n - 1 - (j >> 1) : j >> 1] = KD == PFK_RODFT10 && (j & 1) ? -v : v;
+  } else if constexpr (KD == PFK_REDFT00) {
+    row[j] = v;
+    if (j > 0 && j < n - 1) row[2 * (n - 1) - j] = v;
+  } else if constexpr (KD == PFK_RODFT00) {   // 0, x_0 .. x_(n-1), 0, -x_(n-1) .. -x_0
+    row[j + 1] = v;
+    row[2 * (n + 1) - j - 1] = -v;
+    if (j == 0) row[0] = row[n + 1] = (T)0;
+  } else if constexpr (KD == PFK_REDFT01 || KD == PFK_RODFT01) {
+    const int i = KD == PFK_RODFT01 ? n - 1 - j : j;
+    if (i <= M) row[2 * i] = v;
+    if (i >= M) row[2 * (n - i) + 1] = v;
+    if (i == 0) row[1] = (T)0;
+  } else {
+    const int i = KD == PFK_RODFT11 ? n - 1 - j : j;
+    row[(i & 1) ? n - i : i] = v;
+  }
+}
+
+// mode 1, in place on the staged rows: V_j = e^(i pi j/(2n)) (x'_j - i x'_(n-j)),
+// Im of V_0 and V_M dropped as a c2r drops them, then the c2r combine
+// z_q = (V_q + conj V_(M-q)) + i W_n^q (V_q - conj V_(M-q)) for q and M - q
+template <typename T>
+__device__ __forceinline__ void r2r_spectrum(const MixCtx<T> &X) {
+  const MixGeo &G = X.G;
+  const int M = G.m, total = G.C * (M / 2 + 1), NT = blockDim.x;
+  const C2<T> *tw2 = reinterpret_cast<const C2<T> *>(X.P.tw2);
+  const C2<T> *rtw = reinterpret_cast<const C2<T> *>(X.P.rtw);
+  for (int i = X.tid; i < total; i += NT) {
+    const int c = i & (G.C - 1), q = i >> G.logC, r = M - q;
+    C2<T> *row = X.lds + mix_slot(G, c, 0);
+    const C2<T> xq = row[q], xr = row[r], tq = tw2[q], tr = tw2[r], wq = rtw[q], wr = rtw[r];
+    C2<T> a = cmul(C2<T>{tq.x, -tq.y}, C2<T>{xq.x, -xq.y});
+    C2<T> b = cmul(C2<T>{tr.x, -tr.y}, C2<T>{xr.x, -xr.y});
+    if (q == 0) a.y = b.y = (T)0;
+    const C2<T> wd = cmul(wq, C2<T>{a.x - b.x, a.y + b.y});
+    row[q] = C2<T>{a.x + b.x - wd.y, a.y - b.y + wd.x};
+    if (q > 0 && q < r) {
+      const C2<T> we = cmul(wr, C2<T>{b.x - a.x, b.y + a.y});
+      row[r] = C2<T>{b.x + a.x - we.y, b.y - a.y + we.x};
+    }
+  }
+  lds_barrier();
+}
+
+// the kind's outputs from the inner transform in LDS
+template <int KD, typename T>
+__device__ __forceinline__ void r2r_post(const MixCtx<T> &X) {
+  const pfk_pass &P = X.P;
+  const MixGeo &G = X.G;
+  const int n = (int)P.n, M = G.m, zout = (int)P.zout, nout = (int)P.nout, NT = blockDim.x;
+  constexpr int mode = r2r_mode_of(KD), U = 4;
+  const C2<T> *tw2 = reinterpret_cast<const C2<T> *>(P.tw2);
+  const C2<T> *rtw = reinterpret_cast<const C2<T> *>(P.rtw);
+  auto z = [&](int c, int m) {
+    C2<T> v = X.lds[mix_slot(G, c, m)];
+    v.y *= X.cj;
+    return v;
+  };
+  auto emit = [&](int c, int kk, T y) {
+    const int k = kk - zout;
+    if (k >= 0 && k < nout && c < X.nl)
+      X.dst[X.dof[c] + (int64_t)k * P.sout] = y * msign<T>(P.omod, k);
+  };
+  // items: mode 0 the bins m <= M of the real line, each the outputs of m and of
+  // its mirror; modes 1 and 2 the kept outputs
+  const int cnt = mode == 0 ? M + 1 : nout, total = G.C * cnt;
+  for (int b = X.tid; b < total; b += U * NT) {
+    int cc[U], mm[U];
+    C2<T> w[U], t1[U], t2[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = b + u * NT < total ? b + u * NT : b;
+      cc[u] = G.lm_st ? div_m(i, G.mstore) : i & (G.C - 1);
+      mm[u] = G.lm_st ? i - cc[u] * cnt : i >> G.logC;
+      if constexpr (mode == 0) {
+        w[u] = rtw[mm[u]];
+        if constexpr (KD == PFK_REDFT10 || KD == PFK_RODFT10) {
+          t1[u] = tw2[mm[u]];
+          t2[u] = tw2[n - mm[u]];
+        }
+      } else if constexpr (mode == 2) {
+        const int kk = mm[u] + zout;
+        t1[u] = tw2[4 * ((kk & 1) ? (n - 1 - kk) / 2 : kk / 2)];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (b + u * NT >= total) break;
+      const int c = cc[u], m = mm[u];
+      if constexpr (mode == 0) {
+        // V_m = E_m + W^m O_m from Z_m and conj Z_(M-m)
+        const C2<T> a = z(c, m == M ? 0 : m), b0 = z(c, m == 0 ? 0 : M - m);
+        const C2<T> bb{b0.x, -b0.y};
+        const C2<T> e{(a.x + bb.x) * (T)0.5, (a.y + bb.y) * (T)0.5};
+        const C2<T> o{(a.y - bb.y) * (T)0.5, -(a.x - bb.x) * (T)0.5};
+        C2<T> v = cmul(w[u], o);
+        v = C2<T>{v.x + e.x, v.y + e.y};
+        const bool two = m > 0 && m < M;   // the mirror bin 2M - m has conj V_m
+        if constexpr (KD == PFK_DHT) {
+          emit(c, m, v.x - v.y);
+          if (two) emit(c, n - m, v.x + v.y);
+        } else if constexpr (KD == PFK_REDFT10) {
+          emit(c, m, 2 * cmul(t1[u], v).x);
+          if (two) emit(c, n - m, 2 * cmul(t2[u], C2<T>{v.x, -v.y}).x);
+        } else if constexpr (KD == PFK_RODFT10) {   // reversed
+          emit(c, n - 1 - m, 2 * cmul(t1[u], v).x);
+          if (two) emit(c, m - 1, 2 * cmul(t2[u], C2<T>{v.x, -v.y}).x);
+        } else if constexpr (KD == PFK_REDFT00) {
+          emit(c, m, v.x);
+        } else if (two) {   // RODFT00: n = M - 1 outputs
+          emit(c, m - 1, -v.y);
+        }
+      } else if constexpr (mode == 1) {   // y_2m = v_m, y_(2m+1) = v_(n-1-m), v the real line
+        const int kk = m + zout, idx = (kk & 1) ? n - 1 - (kk - 1) / 2 : kk / 2;
+        const C2<T> v = z(c, idx / 2);
+        const T y = (idx & 1) ? v.y : v.x;
+        emit(c, kk, KD == PFK_RODFT01 && (kk & 1) ? -y : y);   // DST-III: (-1)^k
+      } else {   // u_j = Z_j W_8n^(4j); y_2j = 2 Re u_j, y_(n-1-2j) = -2 Im u_j
+        const int kk = m + zout, j = (kk & 1) ? (n - 1 - kk) / 2 : kk / 2;
+        const C2<T> v = cmul(z(c, j), t1[u]);
+        const T y = (kk & 1) ? -2 * v.y : 2 * v.x;
+        emit(c, kk, KD == PFK_RODFT11 && (kk & 1) ? -y : y);   // DST-IV: (-1)^k
+      }
+    }
+  }
+}
+
+// the first stage of these passes reads the staged tile, the last one leaves
+// its result there
+template <int KIND>
+__device__ __forceinline__ bool mix_packed(const pfk_pass &P) {
+  return mix_r2r(KIND) || (KIND == PFK_C2R && !(P.n & 1));
+}
+template <int KIND>
+__device__ __forceinline__ bool mix_combined(const pfk_pass &P) {
+  return mix_r2r(KIND) || (KIND == PFK_R2C && !(P.n & 1));
+}
+// element p of a staged line
+template <typename T, int KIND>
+__device__ __forceinline__ C2<T> mix_staged(const MixCtx<T> &X, const int c, const int p) {
+  if constexpr (mix_r2r(KIND)) {
+    C2<T> v = X.lds[mix_slot(X.G, c, p)];
+    if constexpr (r2r_mode_of(mix_r2r_kind(KIND)) == 2)   // times W_8n^(4p+1)
+      v = cmul(v, reinterpret_cast<const C2<T> *>(X.P.tw2)[4 * p + 1]);
+    v.y *= X.cj;
+    return v;
+  } else {
+    return c2r_pack(X, c, p);
+  }
+}
+
 // one stage of a codelet radix
 template <typename T, int KIND, int R>
 __device__ __forceinline__ void mix_stage(const MixCtx<T> &X, const int s) {
   constexpr int I = mix_items<R>();
   const MixGeo &G = X.G;
   const bool first = s == 0, last = s == G.nst - 1;
-  const bool packed = KIND == PFK_C2R && !(X.P.n & 1);   // first stage reads LDS too
-  const bool z_lds = KIND == PFK_R2C && !(X.P.n & 1);    // last stage writes LDS too
+  const bool packed = mix_packed<KIND>(X.P), z_lds = mix_combined<KIND>(X.P);
   const int NB = G.nb[s], L = G.len[s], items = NB * G.C;
   const bool lm = first ? G.lm_ld : G.lm_st;
   const C2<T> *tw = X.tw + G.off[s];
@@ -181,7 +366,7 @@ __device__ __forceinline__ void mix_stage(const MixCtx<T> &X, const int s) {
   int cs[I], bs[I], ks[I];
 #pragma unroll
   for (int i = 0; i < I; ++i) {
-    const int it0 = (int)threadIdx.x + i * (int)blockDim.x;
+    const int it0 = X.tid + i * (int)blockDim.x;
     const int it = it0 < items ? it0 : 0;
     if (lm) {
       cs[i] = div_m(it, G.mnb[s]);
@@ -193,7 +378,7 @@ __device__ __forceinline__ void mix_stage(const MixCtx<T> &X, const int s) {
     ks[i] = last ? bs[i] : bs[i] - div_m(bs[i], G.mlen[s]) * L;
     if (it0 >= items) cs[i] = G.C;   // no store (below and in mix_store: c >= nl)
   }
-  if (first && !packed && KIND != PFK_C2R && (G.plain || G.vec)) {
+  if (first && !packed && KIND != PFK_C2R && !mix_r2r(KIND) && (G.plain || G.vec)) {
     // every position present, no modulation: one address per butterfly and a
     // uniform step
     const int64_t sin = KIND == PFK_C2C ? X.P.sin : 1, step = NB * sin;
@@ -225,7 +410,7 @@ __device__ __forceinline__ void mix_stage(const MixCtx<T> &X, const int s) {
     for (int i = 0; i < I; ++i)
 #pragma unroll
       for (int r = 0; r < R; ++r)
-        v[i][r] = c2r_pack(X, cs[i] < G.C ? cs[i] : 0, bs[i] + r * NB);
+        v[i][r] = mix_staged<T, KIND>(X, cs[i] < G.C ? cs[i] : 0, bs[i] + r * NB);
   } else {
 #pragma unroll
     for (int i = 0; i < I; ++i) {
@@ -286,8 +471,7 @@ __device__ __forceinline__ void mix_big(const MixCtx<T> &X, const int s) {
   typedef T v4 __attribute__((ext_vector_type(4)));
   const MixGeo &G = X.G;
   const bool first = s == 0, last = s == G.nst - 1;
-  const bool packed = KIND == PFK_C2R && !(X.P.n & 1);
-  const bool z_lds = KIND == PFK_R2C && !(X.P.n & 1);
+  const bool packed = mix_packed<KIND>(X.P), z_lds = mix_combined<KIND>(X.P);
   const int R = G.rad[s], NB = G.nb[s], L = G.len[s], H = (R - 1) / 2, NT = blockDim.x;
   const C2<T> *tw = X.tw + G.off[s], *tr = X.tw + G.offr[s];
   // pair sums A_r at position r*NB + b, differences B_r at (R-r)*NB + b of the
@@ -295,7 +479,7 @@ __device__ __forceinline__ void mix_big(const MixCtx<T> &X, const int s) {
   constexpr int U = 4;
   const int cnt = (H + 1) * NB, total = G.C * cnt;
   const bool lm = first && !packed && G.lm_ld;
-  for (int i0 = threadIdx.x; i0 < total; i0 += U * NT) {
+  for (int i0 = X.tid; i0 < total; i0 += U * NT) {
     C2<T> x[U], y[U];
     int cc[U], pp[U], mm[U];
 #pragma unroll
@@ -314,8 +498,8 @@ __device__ __forceinline__ void mix_big(const MixCtx<T> &X, const int s) {
         x[u] = mix_load<T, KIND>(X, cc[u], pp[u]);
         y[u] = mix_load<T, KIND>(X, cc[u], mm[u]);
       } else if (first) {
-        x[u] = c2r_pack(X, cc[u], pp[u]);
-        y[u] = c2r_pack(X, cc[u], mm[u]);
+        x[u] = mix_staged<T, KIND>(X, cc[u], pp[u]);
+        y[u] = mix_staged<T, KIND>(X, cc[u], mm[u]);
       } else {
         const int k = b - div_m(b, G.mlen[s]) * L;
         x[u] = X.lds[mix_slot(G, cc[u], pp[u])];
@@ -338,9 +522,9 @@ __device__ __forceinline__ void mix_big(const MixCtx<T> &X, const int s) {
   // Y_q and Y_(R-q), q <= H: a wave takes one butterfly of 8 lines and 16
   // values of q.  Operand columns are (line, re/im); the table operand is
   // W_R^(q r mod R), its index advanced by 4 q per step of 4 r.
-  const int lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4, part = col >> 3;
+  const int lane = X.tid & 63, col = lane & 15, kq = lane >> 4, part = col >> 3;
   const int MT = (H + 16) / 16, LG = G.C >> 3, units = NB * LG * MT;
-  for (int un = threadIdx.x >> 6; un < units; un += NT >> 6) {
+  for (int un = X.tid >> 6; un < units; un += NT >> 6) {
     const int mt = un % MT, v = un / MT, g = v % LG, b = v / LG;
     const int c = g * 8 + (col & 7), q = mt * 16 + col;
     const T *row = reinterpret_cast<const T *>(X.lds2 + mix_slot(G, c, b)) + part;
@@ -375,8 +559,8 @@ __device__ __forceinline__ void mix_big(const MixCtx<T> &X, const int s) {
   }
   lds_barrier();
   if (!last || z_lds) return;
-  const int nf = (int)X.P.nf;
-  for (int i = threadIdx.x; i < G.C * nf; i += NT) {
+  const int nf = G.m;
+  for (int i = X.tid; i < G.C * nf; i += NT) {
     const int c = G.lm_st ? div_m(i, G.mrow) : i & (G.C - 1);
     const int p = G.lm_st ? i - c * nf : i >> G.logC;
     mix_store<T, KIND>(X, c, p, X.lds[mix_slot(G, c, p)]);
@@ -450,8 +634,14 @@ __device__ __forceinline__ void mixed_tile(const pfk_pass &P, const MixGeo &G,
   if (G.text != P.text) left = P.text - line0 % G.text;
   const int nl = left < G.C ? (int)left : G.C;
   mix_lines(P, G.C, G.text, line0, nl, so, dof);
+  // r2r: opaque per tile, else what depends on the thread index alone (table
+  // entries, addresses) is hoisted out of the tile loop and spilled; the other
+  // kinds gain from the hoisting (r2c 210x196x330 complex64 195 us, 206 opaque)
+  int tid = threadIdx.x;
+  if constexpr (mix_r2r(KIND)) asm volatile("" : "+v"(tid));
   MixCtx<T> X{P, G, nl, so, dof, src, dst, tw, reinterpret_cast<C2<T> *>(off0 + 4 * G.C),
-              reinterpret_cast<C2<T> *>(off0 + 4 * G.C) + (BIG ? G.C * G.pitch : 0), P.sign < 0 ? (T)1 : (T)-1};
+              reinterpret_cast<C2<T> *>(off0 + 4 * G.C) + (BIG ? G.C * G.pitch : 0), tid,
+              (mix_r2r(KIND) ? pfk_r2r_mode(P.r2r) != 1 : P.sign < 0) ? (T)1 : (T)-1};
   const bool even = !(P.n & 1);
   const int h = (int)P.nf;
   if (KIND == PFK_C2R && even) {
@@ -459,7 +649,7 @@ __device__ __forceinline__ void mixed_tile(const pfk_pass &P, const MixGeo &G,
     // weights), 128 bytes of loads in flight per thread
     constexpr int U = sizeof(T) == 8 ? 8 : 16;
     const int cnt = h + 1, total = G.C * cnt, NT = blockDim.x;
-    for (int b = threadIdx.x; b < total; b += U * NT) {
+    for (int b = tid; b < total; b += U * NT) {
       C2<T> v[U];
       int cc[U], kk[U];
 #pragma unroll
@@ -488,6 +678,38 @@ __device__ __forceinline__ void mixed_tile(const pfk_pass &P, const MixGeo &G,
     }
     lds_barrier();
   }
+  if constexpr (mix_r2r(KIND)) {
+    // the real lines into their rows, zeros outside the embed
+    constexpr int U = 8;
+    const int cnt = (int)P.n, total = G.C * cnt, NT = blockDim.x;
+    T *rows = reinterpret_cast<T *>(X.lds);
+    for (int b = tid; b < total; b += U * NT) {
+      T v[U];
+      auto at = [&](int u, int &c, int &j) {
+        const int i = b + u * NT < total ? b + u * NT : b;
+        c = G.lm_ld ? div_m(i, G.mload) : i & (G.C - 1);
+        j = G.lm_ld ? i - c * cnt : i >> G.logC;
+      };
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        int c, j0;
+        at(u, c, j0);
+        const int j = j0 - (int)P.zin;
+        v[u] = src[so[c] + (int64_t)(j >= 0 && j < (int)P.nin ? j : 0) * P.sin];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        int c, j0;
+        at(u, c, j0);
+        const int j = j0 - (int)P.zin;
+        const bool ok = j >= 0 && j < (int)P.nin;
+        r2r_put<mix_r2r_kind(KIND)>(rows + 2 * G.pitch * c, cnt, G.m, j0,
+                                    ok ? v[u] * msign<T>(P.imod, j) : (T)0);
+      }
+    }
+    lds_barrier();
+    if constexpr (r2r_mode_of(mix_r2r_kind(KIND)) == 1) r2r_spectrum(X);
+  }
   for (int s = 0; s < G.nst; ++s) {
     switch (G.rad[s]) {
       case 2: mix_stage<T, KIND, 2>(X, s); break;
@@ -510,13 +732,14 @@ __device__ __forceinline__ void mixed_tile(const pfk_pass &P, const MixGeo &G,
         break;
     }
   }
+  if constexpr (mix_r2r(KIND)) r2r_post<mix_r2r_kind(KIND)>(X);
   if (KIND == PFK_R2C && even) {
     // half-spectrum combine: X_k = E_k + W_n^k O_k, U outputs per thread at a
     // time so that their table loads overlap
     constexpr int U = 4;
     const C2<T> *rtw = reinterpret_cast<const C2<T> *>(P.rtw);
     const int cnt = (int)P.nout, total = G.C * cnt, NT = blockDim.x;
-    for (int b = threadIdx.x; b < total; b += U * NT) {
+    for (int b = tid; b < total; b += U * NT) {
       C2<T> w[U];
       int cc[U], kk[U];
 #pragma unroll

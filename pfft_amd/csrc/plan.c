@@ -754,6 +754,8 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
         goto fail;
       }
       ps->work = p->work[k];
+    } else if (ps->r2r_path && (pfk_pass_kernels(ps) & PFK_HAS_MIXED)) {
+      /* one launch, no work arrays */
     } else if (ps->r2r_path) {
       pfk_pass in;
       int64_t l1, l2;
@@ -1206,7 +1208,8 @@ int pa_plan_npasses(const pa_plan *p) { return p ? p->npass : 0; }
 static const char *kernel_name(const pfk_pass *ps) {
   if (ps->kind == PFK_COPY) return "copy";
   if (ps->n1) return "long-two-step";
-  if (ps->r2r_path) return "r2r-inner-fft";
+  if (ps->r2r_path)
+    return (pfk_pass_kernels(ps) & PFK_HAS_MIXED) ? "r2r-mixed" : "r2r-inner-fft";
   const int fam = pfk_pass_kernels(ps);
   const int lm = (ps->variant & 8) && ps->variant != 9 && ps->kind != PFK_R2R &&
                  (ps->prec == PFK_F32 || pfk_pass_plain(ps));

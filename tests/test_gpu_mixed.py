@@ -94,3 +94,41 @@ def test_named():
     names = [ln.split("kernel=")[-1] for ln in pl.describe()]
     pl.destroy()
     assert names.count("mixed") == 2, names
+
+
+# ---- r2r lines as one launch (even inner length) ----
+KINDS = {"DHT": P.DHT, "REDFT00": P.REDFT00, "REDFT01": P.REDFT01, "REDFT10": P.REDFT10,
+         "REDFT11": P.REDFT11, "RODFT00": P.RODFT00, "RODFT01": P.RODFT01,
+         "RODFT10": P.RODFT10, "RODFT11": P.RODFT11}
+# even lengths with codelet and matrix-core inner lengths; the 00 kinds have the
+# inner lengths n - 1 and n + 1, of any parity
+R2R_LENGTHS = [8, 10, 14, 18, 22, 34, 62, 64, 100, 128, 250, 256, 640, 1100]
+R2R_ODD = [9, 13, 17, 33, 65, 129]
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_r2r_lines(kind, prec):
+    for n in R2R_LENGTHS + (R2R_ODD if kind.endswith("00") else []):
+        # strided lines on a ragged tile, then contiguous ones
+        for shape in ([3, n, 19], [3, 5, n]):
+            spec = spec_of("r2r", shape, kinds=[P.DHT if d != shape.index(n) else KINDS[kind]
+                                                for d in range(3)])
+            x = random_input(spec, 5)
+            y = run_gpu(spec, x, prec=prec)
+            assert rel_l2(y, oracle_out(spec, x)) < (1e-12 if prec == "f64" else 4e-6), shape
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_r2r_embed_tuple_transposed(kind):
+    spec = spec_of("r2r", [14, 22, 18], [10, 16, 18], [14, 12, 10], kinds=[KINDS[kind]] * 3,
+                   howmany=2, flags=TO)
+    x = random_input(spec, 6)
+    assert rel_l2(run_gpu(spec, x), oracle_out(spec, x)) < 1e-12
+
+
+def test_r2r_named():
+    a = P.DeviceBuffer(8 * 64 * 64 * 64)
+    pl = P.Plan("r2r", [64, 64, 64], a.ptr, a.ptr, comm=comm_for(2), kinds=[P.REDFT10] * 3)
+    assert all(ln.endswith("kernel=r2r-mixed") for ln in pl.describe()), pl.describe()
+    pl.destroy()
