@@ -20,6 +20,7 @@
 #include <string.h>
 #include "pass_tile.hpp"
 #include "small_tile.hpp"
+#include "plane_tile.hpp"
 
 namespace pfk {
 
@@ -69,6 +70,29 @@ k_batch_small(const pfk_task *__restrict__ tasks, const int t0, const int t1,
   }
 }
 
+// plane passes: an item is a plane
+template <typename T>
+__global__ void __launch_bounds__(1024)
+k_batch_plane(const pfk_task *__restrict__ tasks, const int t0, const int t1,
+              const int64_t item0, const int64_t item1) {
+  extern __shared__ unsigned char smem_raw[];
+  for (int64_t g = item0 + blockIdx.x; g < item1; g += gridDim.x) {
+    const pfk_task &tk = tasks[find_task(tasks, t0, t1, g)];
+    const pfk_pass &P = tk.pass;
+    const PlaneGeo &G = *reinterpret_cast<const PlaneGeo *>(tk.plane);
+    int64_t u = g - tk.first_item, s = 0, d = 0;
+    for (int i = 0; i < P.nb; ++i) {
+      const int64_t k = u % P.bext[i];
+      u /= P.bext[i];
+      s += k * P.bsin[i];
+      d += k * P.bsout[i];
+    }
+    plane_tile<T>(G, P.sign, (const T *)tk.src + 2 * s, (T *)tk.dst + 2 * d, P.twm, P.pl.twm, true,
+                  smem_raw);
+  }
+}
+static_assert(sizeof(PlaneGeo) <= sizeof(pfk_task::plane), "plane geometry in a task");
+
 // short lengths the batch runs with the short-length kernel: those whose
 // workgroups have 4 waves (the batch launches 256 threads), odd lengths
 // above 16 excepted (one line per lane holds too many registers inside the
@@ -77,9 +101,14 @@ __host__ __device__ constexpr bool batch_small_length(int nf, bool f64) {
   return small_length(nf, f64) && small_threads(nf, f64) == 256 && !(nf > 16 && (nf & 1));
 }
 
-// kernel of a task group: 0 = general, else the short length NF
+// Classes of plane tasks: PFK_PLANE_CLASS + their wave count (1..16), so that the
+// planes of a launch need about the same LDS.
+#define PFK_PLANE_CLASS 239
+
+// kernel of a task group: 0 = general, a plane class, else the short length NF
 template <typename T>
 static const void *batch_kernel(int cls) {
+  if (cls > PFK_PLANE_CLASS) return reinterpret_cast<const void *>(&k_batch_plane<T>);
   if (cls == 0) return reinterpret_cast<const void *>(&k_batch_generic<T>);
   switch (cls) {
 #define PFK_BATCH_SMALL(N) \
@@ -112,7 +141,7 @@ typedef struct {
   const void *kernel;
   int t0, t1;
   int64_t i0, i1;
-  int grid;
+  int grid, threads;
   int level;
   size_t lds;
 } batch_group;
@@ -135,7 +164,7 @@ static int launch_group(const pfk_batch *b, const batch_group *g, hipStream_t s)
   int t0 = g->t0, t1 = g->t1;
   int64_t i0 = g->i0, i1 = g->i1;
   void *args[] = {(void *)&tasks, (void *)&t0, (void *)&t1, (void *)&i0, (void *)&i1};
-  hipError_t e = hipLaunchKernel(g->kernel, dim3(grid), dim3(256), args, g->lds, s);
+  hipError_t e = hipLaunchKernel(g->kernel, dim3(grid), dim3(g->threads), args, g->lds, s);
   if (e == hipSuccess) e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_batch launch", e); return 1; }
   return 0;
@@ -196,6 +225,7 @@ static int batch_capture_forked(pfk_batch *b) {
 }
 
 static int task_class(const pfk_task *t) {
+  if (t->pass.pl.n) return PFK_PLANE_CLASS + plane_threads(&t->pass) / 64;
   if (!g_generic_only && t->pass.variant != 1 && t->pass.kind == PFK_C2C &&
       small_covers(&t->pass) && batch_small_length((int)t->pass.nf, t->pass.prec == PFK_F64))
     return (int)t->pass.nf;
@@ -265,7 +295,15 @@ static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task
         int C = -1, pitch = 0;
         size_t ld;
         int64_t nt;
-        if (cls) {
+        if (cls > PFK_PLANE_CLASS) {
+          if (plane_geo(&t->pass, 64 * (cls - PFK_PLANE_CLASS),
+                        reinterpret_cast<PlaneGeo *>(t->plane), &ld)) {
+            set_error_msg("pfk_batch: bad plane pass");
+            return 1;
+          }
+          nt = 1;
+          for (int k = 0; k < t->pass.nb; k++) nt *= t->pass.bext[k];
+        } else if (cls) {
           int64_t lines = t->pass.text;
           for (int k = 0; k < t->pass.nb; k++) lines *= t->pass.bext[k];
           const int lpt = small_lines_per_tile(cls, prec == PFK_F64);
@@ -288,8 +326,15 @@ static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task
       g->lds = lds;
       g->kernel = (prec == PFK_F64) ? batch_kernel<double>(cls) : batch_kernel<float>(cls);
       if (!g->kernel) { set_error_msg("pfk_batch: no kernel"); return 1; }
+      g->threads = cls > PFK_PLANE_CLASS ? 64 * (cls - PFK_PLANE_CLASS) : 256;
+      if (lds > 65536) {
+        const hipError_t e0 = hipFuncSetAttribute(
+            g->kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e0 != hipSuccess) { set_error("pfk_batch LDS", e0); return 1; }
+      }
       int occ = 0;
-      hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, g->kernel, 256, lds);
+      hipError_t e =
+          hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, g->kernel, g->threads, lds);
       if (e != hipSuccess || occ < 1) occ = 1;
       g->grid = ncu * occ;
       i = j;

@@ -76,6 +76,16 @@ typedef struct pfk_mod {
   int64_t half;
 } pfk_mod;
 
+/* Second dimension of a plane pass (plane_tile.hpp): the pass's own line
+ * (contiguous on both sides, every position present) and n lines of it, sin /
+ * sout apart, are transformed together along both dimensions. */
+typedef struct pfk_plane {
+  int64_t n, sin, sout;   /* n 0: no plane */
+  int32_t mix_n;
+  int32_t mix_rad[PFK_MIX_MAXST];
+  const void *twm;        /* stage table of length n (pfk_pass.twm) */
+} pfk_plane;
+
 typedef struct pfk_pass {
   int32_t kind;       /* enum pfk_kind */
   int32_t prec;       /* enum pfk_prec */
@@ -138,6 +148,7 @@ typedef struct pfk_pass {
   int32_t mix_n;
   int32_t mix_rad[PFK_MIX_MAXST];
   const void *twm;
+  pfk_plane pl;
   /* times of the pass (pfk_stamps; NULL: none): its first workgroup stores
    * the clock to `stamp` when it starts, the last PFK_STAMP_ENDS workgroups
    * store it to stamp_end[...] when they end */
@@ -244,11 +255,12 @@ typedef struct pfk_task {
   pfk_pass pass;
   const void *src;
   void *dst;
-  int32_t C, pitch;       /* filled by pfk_batch_create (C < 0: short-length kernel) */
+  int32_t C, pitch;       /* filled by pfk_batch_create (C < 0: short-length or plane kernel) */
   int64_t ntiles;         /* filled by pfk_batch_create */
   int64_t first_item;     /* filled by pfk_batch_create */
   int32_t dep;
   int32_t pad;
+  int64_t plane[36];      /* plane passes: their launch geometry, filled by pfk_batch_create */
 } pfk_task;
 
 /* Batched execution of many passes: tasks grouped by pass level, one
@@ -352,6 +364,9 @@ int  pfk_pass_kernels(const pfk_pass *p);
 /* 1 if the pass is plain (every input and output position present, no
  * modulation or weights): the instantiations without masks run it */
 int  pfk_pass_plain(const pfk_pass *p);
+
+/* LDS bytes of a plane pass (pl.n set), 0 if it has no kernel. */
+size_t pfk_plane_covers(const pfk_pass *p);
 
 /* Timing helpers on the library stream (HIP events). */
 int  pfk_event_create(void **ev);

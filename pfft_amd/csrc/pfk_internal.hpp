@@ -51,6 +51,7 @@ int launch_generic(const pfk_pass *p, const void *src, void *dst);
 int launch_mfma(const pfk_pass *p, const void *src, void *dst);
 int launch_mfma_chain(const pfk_pass *p, const void *src, void *dst);
 int launch_small(const pfk_pass *p, const void *src, void *dst);
+int launch_plane(const pfk_pass *p, const void *src, void *dst);
 int launch_mixed(const pfk_pass *p, const void *src, void *dst);
 int mixed_covers(const pfk_pass *p);  // 1 if launch_mixed has a kernel for the shape
 int fast_covers(const pfk_pass *p);   // 1 if launch_fast has a kernel for the shape

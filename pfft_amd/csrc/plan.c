@@ -70,6 +70,13 @@ struct pa_plan {
   void *work[PA_MAXRNK];         /* long-line passes: lines * nf complex elements */
   void *work2[PA_MAXRNK];        /* long real-line passes: the same again */
   void *r2rw[2];                 /* r2r passes on the inner real FFT: its input / output */
+  /* The passes as executed where two dimensions share one (fuse_planes): pass
+   * fused[i] does logical dimensions fdim[i][0] and, for a plane, fdim[i][1] */
+  int nfused;
+  int fused_alone;               /* also where the plan runs by itself */
+  pfk_pass fused[2];
+  int fsrc[2], fdst[2], fdim[2][2];
+  int pass_of[PA_MAXRNK];        /* pass of a logical dimension */
   /* execution timer (kernel/timer.c fields): pass k adds its device time
    * to trafo[tslot[k]]; events tev[0..npass] bracket the passes, or, where
    * every pass writes stamps, tev[0] is NULL */
@@ -386,6 +393,80 @@ static int cache_policy(const pfk_pass *ps, int first, int last) {
          (db <= (last ? keep_user : keep_mid) ? PFK_KEEP_DST : 0);
 }
 
+/* Unembedded, unshifted 3-d complex plans whose planes (the two inner dimensions)
+ * fit LDS run in two passes instead of three: the plane and dimension 0.  A
+ * TRANSPOSED_OUT plan does the plane first (dimension 0 writes the transposed
+ * output), the others last. */
+static void fuse_planes(pa_plan *p, const arrgeo *geo, const int *ord) {
+  if (p->rnk_n != 3 || p->howmany != 1 || p->tev[0]) return;
+  int at[3];
+  for (int k = 0; k < 3; k++) {
+    const pfk_pass *ps = &p->pass[k];
+    if (ps->kind != PFK_C2C || ps->n1 || ps->mfma || !pfk_pass_plain(ps)) return;
+    at[ord[k]] = p->pass_of[ord[k]] = k;
+  }
+  const int plane_first = (p->transp & PFFT_TRANSPOSED_OUT) != 0;
+  const arrgeo *inter = &geo[1];
+  for (int i = 0; i < 2; i++) {
+    const arrgeo *S = i ? inter : &p->gin, *D = i ? &p->gout : inter;
+    pfk_pass *q = &p->fused[i];
+    p->fsrc[i] = i ? ROLE_S0 : ROLE_IN;
+    p->fdst[i] = i ? ROLE_OUT : ROLE_S0;
+    INT ss[PA_MAXRNK], sd[PA_MAXRNK];
+    if (i == !plane_first) {
+      const pfk_pass *row = &p->pass[at[2]], *col = &p->pass[at[1]];
+      *q = *row;
+      q->src_elems = geo_strides(S, ss);
+      q->dst_elems = geo_strides(D, sd);
+      if (ss[2] != 1 || sd[2] != 1) return;
+      q->sin = q->sout = 1;
+      q->text = 1;
+      q->tsin = q->tsout = 0;
+      q->nb = 1;
+      q->bext[0] = p->n[0];
+      q->bsin[0] = ss[0];
+      q->bsout[0] = sd[0];
+      q->pl.n = p->n[1];
+      q->pl.sin = ss[1];
+      q->pl.sout = sd[1];
+      q->pl.mix_n = col->mix_n;
+      memcpy(q->pl.mix_rad, col->mix_rad, sizeof q->pl.mix_rad);
+      q->pl.twm = col->twm;
+      if ((p->n[0] - 1) * ss[0] + (p->n[1] - 1) * ss[1] + p->n[2] > q->src_elems ||
+          (p->n[0] - 1) * sd[0] + (p->n[1] - 1) * sd[1] + p->n[2] > q->dst_elems ||
+          !pfk_plane_covers(q))
+        return;
+      p->fdim[i][0] = 2;
+      p->fdim[i][1] = 1;
+    } else {
+      *q = p->pass[at[0]];
+      if (fill_geometry(q, S, D, 0) || check_bounds(q)) return;
+      p->fdim[i][0] = p->fdim[i][1] = 0;
+    }
+    q->variant = 0;
+    q->cache = cache_policy(q, i == 0, i == 1);
+  }
+  p->nfused = 2;
+  /* A plane is a workgroup: by itself a plan needs about as many planes as there
+   * are CUs, and two planes a CU.  Pairs against three passes: complex128
+   * 64x64x64 61 / 53 us, 256x64x64 75 / 80, 300x50x60 84 / 96, 256x16x200 70 /
+   * 85; complex64 1000x100x100 (one plane a CU) 293 / 234, 512x128x128 180 /
+   * 178, 300x50x60 72 / 87. */
+  p->fused_alone = p->n[0] >= 192 && pfk_plane_covers(&p->fused[plane_first ? 0 : 1]) <= 72 * 1024;
+}
+
+/* the passes as executed, fused or one per dimension */
+static int prog_n(const pa_plan *p, int fused) { return fused ? p->nfused : p->npass; }
+static const pfk_pass *prog_pass(const pa_plan *p, int fused, int i) {
+  return fused ? &p->fused[i] : &p->pass[i];
+}
+static int prog_src(const pa_plan *p, int fused, int i) {
+  return fused ? p->fsrc[i] : p->src_role[i];
+}
+static int prog_dst(const pa_plan *p, int fused, int i) {
+  return fused ? p->fdst[i] : p->dst_role[i];
+}
+
 pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const INT *no,
                         INT howmany, const INT *iblock, const INT *oblock, void *in, void *out,
                         MPI_Comm comm, int sign, const int *skip_trafos, unsigned tf,
@@ -555,7 +636,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
   int64_t r2r_elems[2] = {0, 0};   /* reals of the inner-FFT work arrays */
   p->npass = R;
   int src_role = ROLE_IN;
-  arrgeo prev_inter;
+  arrgeo prev_inter, geo[PA_MAXRNK + 1];
   int have_prev = 0;
   for (int k = 0; k < R; k++) {
     const int d = ord[k];
@@ -718,6 +799,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
       }
     }
     if (fill_geometry(ps, &cur, &nxt, d)) goto fail;
+    geo[k + 1] = nxt;
     if (check_bounds(ps)) goto fail;
     if (ps->n1) {
       int64_t lines = ps->text;
@@ -831,6 +913,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
       pa_error("event creation failed: %s", pfk_last_error());
       goto fail;
     }
+  fuse_planes(p, geo, ord);
   tune_plan(p);
   return p;
 fail:
@@ -892,14 +975,15 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
   }
   void *bufs[4] = {din, dout, p->scratch[0], p->scratch[1]};
   int err = p->tev[0] ? pfk_event_record(p->tev[0]) : 0;
-  for (int i = 0; i < p->npass && !err; i++) {
-    const int k = adjoint ? p->npass - 1 - i : i;
-    const pfk_pass *fw = &p->pass[k];
+  const int fused = p->fused_alone, np = prog_n(p, fused);
+  for (int i = 0; i < np && !err; i++) {
+    const int k = adjoint ? np - 1 - i : i;
+    const pfk_pass *fw = prog_pass(p, fused, k);
     pfk_pass a = *fw;
     a.stamp = stamps ? stamps + i : NULL;
-    a.stamp_end = stamps && i == p->npass - 1 ? stamps + PFK_STAMPS - PFK_STAMP_ENDS : NULL;
+    a.stamp_end = stamps && i == np - 1 ? stamps + PFK_STAMPS - PFK_STAMP_ENDS : NULL;
     if (!adjoint) {
-      err = pfk_launch_pass(&a, bufs[p->src_role[k]], bufs[p->dst_role[k]]);
+      err = pfk_launch_pass(&a, bufs[prog_src(p, fused, k)], bufs[prog_dst(p, fused, k)]);
     } else {
       a.sign = -fw->sign;
       a.nin = fw->nout; a.zin = fw->zout;
@@ -908,15 +992,17 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
       a.sin = fw->sout; a.sout = fw->sin;
       a.tsin = fw->tsout; a.tsout = fw->tsin;
       for (int b = 0; b < a.nb; b++) { a.bsin[b] = fw->bsout[b]; a.bsout[b] = fw->bsin[b]; }
+      a.pl.sin = fw->pl.sout; a.pl.sout = fw->pl.sin;
       a.src_elems = fw->dst_elems; a.dst_elems = fw->src_elems;
       if (fw->kind == PFK_R2C) { a.kind = PFK_C2R; a.hw = 1; }
       else if (fw->kind == PFK_C2R) { a.kind = PFK_R2C; a.hw = 2; }
-      a.tw = p->tw_adj[k]; a.rtw = p->rtw_adj[k];
+      if (!fused) { a.tw = p->tw_adj[k]; a.rtw = p->rtw_adj[k]; }
+      else if (!a.pl.n) a.tw = p->tw_adj[p->pass_of[0]];
       a.cache = (fw->cache & PFK_KEEP_SRC ? PFK_KEEP_DST : 0) |
                 (fw->cache & PFK_KEEP_DST ? PFK_KEEP_SRC : 0);
       /* map roles: forward IN <-> adjoint OUT */
       static const int swap_io[4] = {ROLE_OUT, ROLE_IN, ROLE_S0, ROLE_S1};
-      err = pfk_launch_pass(&a, bufs[swap_io[p->dst_role[k]]], bufs[swap_io[p->src_role[k]]]);
+      err = pfk_launch_pass(&a, bufs[swap_io[prog_dst(p, fused, k)]], bufs[swap_io[prog_src(p, fused, k)]]);
     }
     if (!err && p->tev[0]) err = pfk_event_record(p->tev[i + 1]);
     if (err) pa_error("pass %d launch failed: %s", k, pfk_last_error());
@@ -926,10 +1012,15 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
     uint64_t end = 0;
     for (int i = PFK_STAMPS - PFK_STAMP_ENDS; i < PFK_STAMPS; i++)
       if (stamps[i] > end) end = stamps[i];
-    for (int i = 0; i < p->npass; i++) {
-      const int k = adjoint ? p->npass - 1 - i : i;
-      p->timer->trafo[p->tslot[k]] +=
-          pfk_stamp_seconds(stamps[i], i + 1 < p->npass ? stamps[i + 1] : end);
+    for (int i = 0; i < np; i++) {
+      const int k = adjoint ? np - 1 - i : i;
+      const double t = pfk_stamp_seconds(stamps[i], i + 1 < np ? stamps[i + 1] : end);
+      if (!fused) {
+        p->timer->trafo[p->tslot[k]] += t;
+      } else {   /* a plane's time: half to each of its dimensions */
+        p->timer->trafo[p->tslot[p->pass_of[p->fdim[k][0]]]] += 0.5 * t;
+        p->timer->trafo[p->tslot[p->pass_of[p->fdim[k][1]]]] += 0.5 * t;
+      }
     }
   } else if (!err && p->tev[0]) {
     for (int i = 0; i < p->npass; i++) {
@@ -1007,11 +1098,25 @@ static void batch_cache_forget(uint64_t id) {
   }
 }
 
+/* Planes of a batch share its launches: fused where there are enough of them
+ * to fill the GPU several times (batches of uneven complex64 transforms, sides
+ * 24..128, three passes / planes: 16 of them, 1000 planes, 156 / 155 us; 32,
+ * 206 / 171; 128, 602 / 478). */
+static int64_t batch_planes(const pa_plan *const *plans, int count) {
+  int64_t n = 0;
+  for (int i = 0; i < count; i++)
+    if (plans[i]->nfused) n += plans[i]->n[0];
+  return n;
+}
+#define PA_BATCH_PLANES 1024
+
 static pfk_batch *batch_build(const pa_plan *const *plans, int count) {
   int maxp = 0, ntasks = 0;
+  const int fuse = batch_planes(plans, count) >= PA_BATCH_PLANES;
   for (int i = 0; i < count; i++) {
-    if (plans[i]->npass > maxp) maxp = plans[i]->npass;
-    ntasks += plans[i]->npass;
+    const int n = prog_n(plans[i], fuse && plans[i]->nfused);
+    if (n > maxp) maxp = n;
+    ntasks += n;
   }
   pfk_task *tasks = (pfk_task *)calloc((size_t)ntasks, sizeof(pfk_task));
   int *last = (int *)malloc(sizeof(int) * (size_t)count);
@@ -1020,11 +1125,12 @@ static pfk_batch *batch_build(const pa_plan *const *plans, int count) {
   for (int lev = 0; lev < maxp; lev++)
     for (int i = 0; i < count; i++) {
       const pa_plan *p = plans[i];
-      if (lev >= p->npass) continue;
+      const int fused = fuse && p->nfused;
+      if (lev >= prog_n(p, fused)) continue;
       void *bufs[4] = {p->in, p->out, p->scratch[0], p->scratch[1]};
-      tasks[k].pass = p->pass[lev];
-      tasks[k].src = bufs[p->src_role[lev]];
-      tasks[k].dst = bufs[p->dst_role[lev]];
+      tasks[k].pass = *prog_pass(p, fused, lev);
+      tasks[k].src = bufs[prog_src(p, fused, lev)];
+      tasks[k].dst = bufs[prog_dst(p, fused, lev)];
       tasks[k].dep = last[i];
       last[i] = k;
       k++;
@@ -1132,27 +1238,29 @@ int pa_plans_execute_batch_noalloc(const pa_plan *const *plans, int count) {
   /* level order (every plan's pass 0, then every pass 1, ...), each task
    * depending on the previous pass of its plan: within the block of level
    * lev-1 the plans with at least lev passes appear in plan order */
+  const int fuse = batch_planes(plans, count) >= PA_BATCH_PLANES;
   int k = 0, prev_start = 0;
   for (int lev = 0; lev < maxp; lev++) {
     const int cur_start = k;
     int a = prev_start;
     for (int i = 0; i < count; i++) {
       const pa_plan *p = plans[i];
-      const int in_prev = lev > 0 && p->npass > lev - 1;
-      if (lev < p->npass) {
+      const int fused = fuse && p->nfused;
+      const int in_prev = lev > 0 && prog_n(p, fused) > lev - 1;
+      if (lev < prog_n(p, fused)) {
         void *bufs[4] = {p->in, p->out, p->scratch[0], p->scratch[1]};
         pfk_task *t = &g_noalloc_tasks[k++];
         memset(t, 0, sizeof(*t));
-        t->pass = p->pass[lev];
-        t->src = bufs[p->src_role[lev]];
-        t->dst = bufs[p->dst_role[lev]];
+        t->pass = *prog_pass(p, fused, lev);
+        t->src = bufs[prog_src(p, fused, lev)];
+        t->dst = bufs[prog_dst(p, fused, lev)];
         t->dep = lev > 0 ? a : -1;
       }
       if (in_prev) a++;
     }
     prev_start = cur_start;
   }
-  if (pfk_batch_run_noalloc(g_noalloc_tasks, ntasks)) {
+  if (pfk_batch_run_noalloc(g_noalloc_tasks, k)) {
     pa_error("execute_batch_noalloc failed: %s", pfk_last_error());
     return 1;
   }
