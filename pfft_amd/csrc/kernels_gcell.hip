@@ -40,9 +40,24 @@ struct GcDims {
   uint32_t wloc;     // n2 * tuple: reals per local row
 };
 
+// Streaming (nontemporal) or ordinary accesses.  The block's scratch copy is
+// written and read again at once: ordinary accesses leave it in the 256 MB
+// memory-side cache, and streaming the user's array past it leaves it the room
+// (gc_streams).
+template <bool ST, typename T>
+__device__ __forceinline__ T gc_ld(const T *p) {
+  if constexpr (ST) return __builtin_nontemporal_load(p);
+  else return *p;
+}
+template <bool ST, typename T>
+__device__ __forceinline__ void gc_st(T *p, T v) {
+  if constexpr (ST) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // exchange: dst[b] for every box element b <- src (local block) at the
 // periodic source index
-template <typename T>
+template <typename T, bool SS, bool SD>
 __global__ void __launch_bounds__(GC_NT)
 k_gc_fill(const GcDims d, const int64_t total, const T *__restrict__ src, T *__restrict__ dst) {
   const int64_t b0 = (int64_t)blockIdx.x * GC_CH;
@@ -66,12 +81,90 @@ k_gc_fill(const GcDims d, const int64_t total, const T *__restrict__ src, T *__r
     si[j] = (b0 + o < total) ? s : 0;
   }
 #pragma unroll
-  for (int j = 0; j < GC_EPT; j++) v[j] = src[si[j]];
+  for (int j = 0; j < GC_EPT; j++) v[j] = gc_ld<SS>(src + si[j]);
 #pragma unroll
   for (int j = 0; j < GC_EPT; j++) {
     const int64_t b = b0 + (int64_t)(j * GC_NT) + threadIdx.x;
-    if (b < total) dst[b] = v[j];
+    if (b < total) gc_st<SD>(dst + b, v[j]);
   }
+}
+
+// The row copies of exchange (FILL: box rows from their periodic source rows)
+// and of reduce's first part (local rows from their own box rows), a wave per
+// row: the row is decoded once per wave, and along the row the periodic source
+// is one subtraction, where the kernels above spend five integer divisions per
+// element.  For rows of at least a wave.
+template <typename T, bool SS, bool SD, bool FILL>
+__device__ __forceinline__ void gc_rows(const GcDims &d, const T *__restrict__ src,
+                                        T *__restrict__ dst) {
+  constexpr uint32_t U = 16;
+  const uint32_t w = FILL ? d.wbox : d.wloc;
+  const uint32_t rows = FILL ? d.ngc[0] * d.ngc[1] : d.n[0] * d.n[1];
+  const uint32_t lane = threadIdx.x & 63, waves = gridDim.x * (GC_NT / 64);
+  const uint32_t shift = d.off[2] * d.tuple;   // box real e shows local real (e + shift) mod wloc
+  const bool once = d.wbox + shift <= 2 * d.wloc;
+  const uint32_t w0 = __builtin_amdgcn_readfirstlane(blockIdx.x * (GC_NT / 64) + (threadIdx.x >> 6));
+  for (uint64_t r = w0; r < rows; r += waves) {
+    const uint32_t row = (uint32_t)r;
+    const T *a;
+    if constexpr (FILL) {
+      const uint32_t k0 = row / d.ngc[1], k1 = row - k0 * d.ngc[1];
+      const uint32_t s0 = (k0 + d.off[0]) % d.n[0], s1 = (k1 + d.off[1]) % d.n[1];
+      a = src + ((int64_t)s0 * d.n[1] + s1) * d.wloc;
+    } else {
+      const uint32_t i0 = row / d.n[1], i1 = row - i0 * d.n[1];
+      a = src + ((int64_t)(d.gb[0] + i0) * d.ngc[1] + d.gb[1] + i1) * d.wbox + d.gb[2] * d.tuple;
+    }
+    T *o = dst + (int64_t)row * w;
+    for (uint32_t e0 = 0; e0 < w; e0 += 64 * U) {
+      T v[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t e = e0 + 64 * u + lane;
+        uint32_t c = e < w ? e : 0;
+        if constexpr (FILL) {
+          c += shift;
+          if (once) c = c >= d.wloc ? c - d.wloc : c;
+          else c %= d.wloc;
+        }
+        if (e0 + 64 * u < w) v[u] = gc_ld<SS>(a + c);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t e = e0 + 64 * u + lane;
+        if (e < w) gc_st<SD>(o + e, v[u]);
+      }
+    }
+  }
+}
+
+template <typename T, bool SS, bool SD>
+__global__ void __launch_bounds__(GC_NT)
+k_gc_fill_rows(const GcDims d, const T *__restrict__ src, T *__restrict__ dst) {
+  gc_rows<T, SS, SD, true>(d, src, dst);
+}
+
+template <typename T, bool SS, bool SD>
+__global__ void __launch_bounds__(GC_NT)
+k_gc_own_rows(const GcDims d, const T *__restrict__ src, T *__restrict__ dst) {
+  gc_rows<T, SS, SD, false>(d, src, dst);
+}
+
+// Single floats in rows of at least a wave, from 16 MiB on: the linear kernels'
+// divisions bound 4-byte elements (512^3, 4 ghost cells: exchange 515 -> 430 us,
+// reduce 495 -> 438).  With 8-byte elements they hide behind the accesses and the
+// longer contiguous runs of the linear kernels are faster (fill 378 against 409
+// us; float pairs, reduce 509 against 564), and small blocks lose 3 us to the
+// row's scalar arithmetic.
+template <typename T>
+static bool gc_by_rows(const GcDims &d, int64_t nloc) {
+  return sizeof(T) == 4 && d.tuple == 1 && d.wloc >= 64 && nloc >= (int64_t)4 << 20;
+}
+
+// workgroups of a row kernel: a wave per row, at most 2^16 of them
+static int64_t gc_row_blocks(int64_t rows) {
+  const int64_t b = (rows + GC_NT / 64 - 1) / (GC_NT / 64);
+  return b < 65536 ? b : 65536;
 }
 
 // Sum of the images of local index i along one dimension, in the
@@ -100,7 +193,7 @@ __device__ __forceinline__ T gc_chain(uint32_t q, uint32_t n, uint32_t ngc, F f)
 
 // reduce, part 1: out[l] <- the box value at local element l's own
 // position (the whole sum for the elements without further images).
-template <typename T>
+template <typename T, bool SS, bool SD>
 __global__ void __launch_bounds__(GC_NT)
 k_gc_own(const GcDims d, const int64_t total, const T *__restrict__ src, T *__restrict__ out) {
   const int64_t b0 = (int64_t)blockIdx.x * GC_CH;
@@ -124,11 +217,11 @@ k_gc_own(const GcDims d, const int64_t total, const T *__restrict__ src, T *__re
     pos[j] = (int64_t)p0 * s0 + (int64_t)p1 * s1 + (int64_t)(d.gb[2] + i2) * d.tuple + h;
   }
 #pragma unroll
-  for (int j = 0; j < GC_EPT; j++) v[j] = src[pos[j]];
+  for (int j = 0; j < GC_EPT; j++) v[j] = gc_ld<SS>(src + pos[j]);
 #pragma unroll
   for (int j = 0; j < GC_EPT; j++) {
     const int64_t l = b0 + (int64_t)(j * GC_NT) + threadIdx.x;
-    if (l < total) out[l] = v[j];
+    if (l < total) gc_st<SD>(out + l, v[j]);
   }
 }
 
@@ -190,7 +283,7 @@ k_gc_shell(const GcDims d, const GcShell sh, const T *__restrict__ src, T *__res
 
 // reduce, part 3: data[b] <- b < nloc ? loc[b] : 0 over the box (with
 // nloc == total: the block copy of exchange)
-template <typename T>
+template <typename T, bool SS, bool SD>
 __global__ void __launch_bounds__(GC_NT)
 k_gc_compact(const int64_t nloc, const int64_t total, const T *__restrict__ loc,
              T *__restrict__ data) {
@@ -199,13 +292,13 @@ k_gc_compact(const int64_t nloc, const int64_t total, const T *__restrict__ loc,
 #pragma unroll
   for (int j = 0; j < GC_EPT; j++) {
     const int64_t b = b0 + (int64_t)(j * GC_NT) + threadIdx.x;
-    v[j] = loc[b < nloc ? b : 0];
+    v[j] = gc_ld<SS>(loc + (b < nloc ? b : 0));
     if (b >= nloc) v[j] = (T)0;
   }
 #pragma unroll
   for (int j = 0; j < GC_EPT; j++) {
     const int64_t b = b0 + (int64_t)(j * GC_NT) + threadIdx.x;
-    if (b < total) data[b] = v[j];
+    if (b < total) gc_st<SD>(data + b, v[j]);
   }
 }
 
@@ -245,6 +338,29 @@ int gc_event(void *const *ev, int k) {
   return 0;
 }
 
+// Launches the <stream source, stream destination> form of kernel K.
+#define GC_LAUNCH(K, T, ss, sd, blocks, ...)                                                   \
+  do {                                                                                         \
+    const dim3 grid_((unsigned)(blocks)), blk_(GC_NT);                                         \
+    if (ss && sd) hipLaunchKernelGGL((K<T, true, true>), grid_, blk_, 0, g_stream, __VA_ARGS__);        \
+    else if (ss) hipLaunchKernelGGL((K<T, true, false>), grid_, blk_, 0, g_stream, __VA_ARGS__);       \
+    else if (sd) hipLaunchKernelGGL((K<T, false, true>), grid_, blk_, 0, g_stream, __VA_ARGS__);       \
+    else hipLaunchKernelGGL((K<T, false, false>), grid_, blk_, 0, g_stream, __VA_ARGS__);              \
+  } while (0)
+
+// Streaming: the user's array from blocks of 80 MiB on (50 MB blocks lost 4%),
+// the scratch copy where
+// it exceeds what the memory-side cache can hold (288 MiB, as the passes'):
+// exchange and reduce of 256^3 doubles with their two fills 368 -> 355 us,
+// 512^3 doubles 821 / 845 -> 797 / 823.
+struct GcStreams {
+  bool user, scratch;
+};
+static GcStreams gc_streams(int64_t nloc, size_t esz) {
+  const double bytes = (double)nloc * (double)esz;
+  return GcStreams{bytes >= 80.0 * 1048576, bytes > 288.0 * 1048576};
+}
+
 template <typename T>
 int gc_exchange(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   GcDims d;
@@ -252,14 +368,18 @@ int gc_exchange(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   if (gc_dims(g, &d, &L, &G)) return 1;
   if (gc_event(ev, 0)) return 1;
   // block copy: the compact kernel with nothing to zero
-  hipLaunchKernelGGL(k_gc_compact<T>, dim3((unsigned)((L + GC_CH - 1) / GC_CH)), dim3(GC_NT), 0,
-                     g_stream, L, L, (const T *)data, scratch);
+  const GcStreams st = gc_streams(L, sizeof(T));
+  GC_LAUNCH(k_gc_compact, T, st.user, st.scratch, (L + GC_CH - 1) / GC_CH, L, L, (const T *)data,
+            scratch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_gc_exchange copy", e); return 1; }
   if (gc_event(ev, 1)) return 1;
   const int64_t nb = (G + GC_CH - 1) / GC_CH;
-  hipLaunchKernelGGL(k_gc_fill<T>, dim3((unsigned)nb), dim3(GC_NT), 0, g_stream, d, G,
-                     (const T *)scratch, data);
+  if (gc_by_rows<T>(d, L))
+    GC_LAUNCH(k_gc_fill_rows, T, st.scratch, st.user, gc_row_blocks(g->ngc[0] * g->ngc[1]), d,
+              (const T *)scratch, data);
+  else
+    GC_LAUNCH(k_gc_fill, T, st.scratch, st.user, nb, d, G, (const T *)scratch, data);
   e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_gc_exchange", e); return 1; }
   return gc_event(ev, 2);
@@ -285,8 +405,13 @@ int gc_reduce(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   sh.c1 = I[0] * E[1] * g->n[2] * g->tuple;
   sh.c2 = I[0] * I[1] * E[2] * g->tuple;
   if (gc_event(ev, 0)) return 1;
-  hipLaunchKernelGGL(k_gc_own<T>, dim3((unsigned)((L + GC_CH - 1) / GC_CH)), dim3(GC_NT), 0,
-                     g_stream, d, L, (const T *)data, scratch);
+  const GcStreams st = gc_streams(L, sizeof(T));
+  if (gc_by_rows<T>(d, L))
+    GC_LAUNCH(k_gc_own_rows, T, st.user, st.scratch, gc_row_blocks(g->n[0] * g->n[1]), d,
+              (const T *)data, scratch);
+  else
+    GC_LAUNCH(k_gc_own, T, st.user, st.scratch, (L + GC_CH - 1) / GC_CH, d, L, (const T *)data,
+              scratch);
   hipError_t e = hipGetLastError();
   const int64_t nshell = sh.c0 + sh.c1 + sh.c2;
   if (e == hipSuccess && nshell > 0) {
@@ -296,8 +421,8 @@ int gc_reduce(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   }
   if (e != hipSuccess) { set_error("pfk_gc_reduce sum", e); return 1; }
   if (gc_event(ev, 1)) return 1;
-  hipLaunchKernelGGL(k_gc_compact<T>, dim3((unsigned)((G + GC_CH - 1) / GC_CH)), dim3(GC_NT), 0,
-                     g_stream, L, G, (const T *)scratch, data);
+  GC_LAUNCH(k_gc_compact, T, st.scratch, st.user, (G + GC_CH - 1) / GC_CH, L, G,
+            (const T *)scratch, data);
   e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_gc_reduce compact", e); return 1; }
   return gc_event(ev, 2);
