@@ -920,7 +920,7 @@ int pfk_launch_pass(const pfk_pass *p, const void *src, void *dst) {
 
 int pfk_pass_stamps(const pfk_pass *p) {
   if (p->kind == PFK_R2R && p->r2r_path) return !g_generic_only && mixed_covers(p);
-  return !p->n1 && !p->mfma;
+  return !p->n1;
 }
 
 #define STAMP_BLOCKS 64

@@ -75,6 +75,7 @@ k_c2c_mfma(const pfk_pass P, const int64_t tile_base, const float *__restrict__ 
   constexpr int A = LG / 4;          // radix-16 MFMA stages
   constexpr int RL = 1 << (LG % 4);  // last VALU stage radix (1: none)
   __shared__ f2 lds[NF * C];
+  stamp_begin(P);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int jj = lane & 15, qq = lane >> 4;
@@ -293,6 +294,7 @@ k_c2c_mfma(const pfk_pass P, const int64_t tile_base, const float *__restrict__ 
     const float f = msign_m(P.omod, k) * unscale;
     d[db + (int64_t)c * P.tsout + (int64_t)k * P.sout] = f2{v.x * f, v.y * f};
   }
+  stamp_end(P);
 }
 
 // ---------------------------------------------------------------------------
@@ -406,6 +408,7 @@ k_c2c_mfma_reg(const pfk_pass P, const int64_t item0, const int64_t item_end,
   constexpr int RL = 1 << (LG % 4);  // last VALU stage radix (1: none)
   __shared__ f2 lds[LM ? C * (NF + NF / 16) : NF * C];
   __shared__ f2 twl[NF];
+  stamp_begin(P);
   const int tid = threadIdx.x;
   twl[tid] = reinterpret_cast<const f2 *>(P.tw)[tid];
   const int zin = (int)P.zin, nin = (int)P.nin, zout = (int)P.zout, nout = (int)P.nout;
@@ -591,6 +594,7 @@ k_c2c_mfma_reg(const pfk_pass P, const int64_t item0, const int64_t item_end,
   lds_barrier();   // twiddle table
   while (step(xa, xb) && step(xb, xa)) {
   }
+  stamp_end(P);
 }
 
 template <int NF, int MODE, int SIGN, bool LM>

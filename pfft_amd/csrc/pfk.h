@@ -384,8 +384,7 @@ int  pfk_event_destroy(void *ev);
 #define PFK_STAMPS 48
 uint64_t *pfk_stamps(void);
 double pfk_stamp_seconds(uint64_t from, uint64_t to);
-/* 1 if the kernels that run the pass write its stamps (single launch, not the
- * MFMA forms) */
+/* 1 if the kernels that run the pass write its stamps (single launch) */
 int  pfk_pass_stamps(const pfk_pass *p);
 
 /* Complex conjugation / scaling utility kernels on device arrays. */
