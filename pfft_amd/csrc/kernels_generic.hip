@@ -37,11 +37,11 @@ void set_error_msg(const char *msg) { snprintf(g_err, sizeof(g_err), "%s", msg);
 template <typename T, int KIND, int EPT>
 __global__ void __launch_bounds__(256)
 k_pass_generic(const pfk_pass P, const int C, const int pitch, const int64_t tile_base,
-               const T *__restrict__ src, T *__restrict__ dst) {
+               const int64_t ntiles, const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
-  stamp_begin(P);
+  stamp_begin(P, tile_base + blockIdx.x);
   pass_tile<T, KIND, EPT>(P, C, pitch, tile_base + blockIdx.x, src, dst, smem_raw);
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - tile_base - blockIdx.x);
 }
 
 // number of complex LDS slots one line needs
@@ -90,23 +90,23 @@ static int launch_generic_t(const pfk_pass *p, const void *src, void *dst) {
     switch (p->kind) {
       case PFK_C2C:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_C2C, EPT>), grid, block, lds, g_stream, *p, C,
-                           (int)pitch, base, s, d);
+                           (int)pitch, base, ntiles, s, d);
         break;
       case PFK_R2C:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_R2C, EPT>), grid, block, lds, g_stream, *p, C,
-                           (int)pitch, base, s, d);
+                           (int)pitch, base, ntiles, s, d);
         break;
       case PFK_C2R:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_C2R, EPT>), grid, block, lds, g_stream, *p, C,
-                           (int)pitch, base, s, d);
+                           (int)pitch, base, ntiles, s, d);
         break;
       case PFK_R2R:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_R2R, EPT>), grid, block, lds, g_stream, *p, C,
-                           (int)pitch, base, s, d);
+                           (int)pitch, base, ntiles, s, d);
         break;
       default:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_COPY, EPT>), grid, block, lds, g_stream, *p, C,
-                           (int)pitch, base, s, d);
+                           (int)pitch, base, ntiles, s, d);
         break;
     }
     hipError_t e = hipGetLastError();

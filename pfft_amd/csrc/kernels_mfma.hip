@@ -68,14 +68,14 @@ __device__ __forceinline__ f2 w16(int m, int sign) {
 
 template <int NF, int C, int MODE, int SIGN>
 __global__ void __launch_bounds__(512)
-k_c2c_mfma(const pfk_pass P, const int64_t tile_base, const float *__restrict__ src,
-           float *__restrict__ dst) {
+k_c2c_mfma(const pfk_pass P, const int64_t tile_base, const int64_t ntiles,
+           const float *__restrict__ src, float *__restrict__ dst) {
   constexpr int NT = 512;
   constexpr int LG = (NF == 256) ? 8 : (NF == 512) ? 9 : (NF == 1024) ? 10 : (NF == 2048) ? 11 : 12;
   constexpr int A = LG / 4;          // radix-16 MFMA stages
   constexpr int RL = 1 << (LG % 4);  // last VALU stage radix (1: none)
   __shared__ f2 lds[NF * C];
-  stamp_begin(P);
+  stamp_begin(P, tile_base + blockIdx.x);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int jj = lane & 15, qq = lane >> 4;
@@ -294,7 +294,7 @@ k_c2c_mfma(const pfk_pass P, const int64_t tile_base, const float *__restrict__ 
     const float f = msign_m(P.omod, k) * unscale;
     d[db + (int64_t)c * P.tsout + (int64_t)k * P.sout] = f2{v.x * f, v.y * f};
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - tileid);
 }
 
 // ---------------------------------------------------------------------------
@@ -408,7 +408,7 @@ k_c2c_mfma_reg(const pfk_pass P, const int64_t item0, const int64_t item_end,
   constexpr int RL = 1 << (LG % 4);  // last VALU stage radix (1: none)
   __shared__ f2 lds[LM ? C * (NF + NF / 16) : NF * C];
   __shared__ f2 twl[NF];
-  stamp_begin(P);
+  stamp_begin(P, item0 + blockIdx.x);
   const int tid = threadIdx.x;
   twl[tid] = reinterpret_cast<const f2 *>(P.tw)[tid];
   const int zin = (int)P.zin, nin = (int)P.nin, zout = (int)P.zout, nout = (int)P.nout;
@@ -594,7 +594,7 @@ k_c2c_mfma_reg(const pfk_pass P, const int64_t item0, const int64_t item_end,
   lds_barrier();   // twiddle table
   while (step(xa, xb) && step(xb, xa)) {
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - item);
 }
 
 template <int NF, int MODE, int SIGN, bool LM>
@@ -654,10 +654,10 @@ static int launch_mfma_nf(const pfk_pass *p, const void *src, void *dst) {
     const int64_t nblk = (ntiles - base) < chunk ? (ntiles - base) : chunk;
     if (p->sign < 0)
       hipLaunchKernelGGL((k_c2c_mfma<NF, C, MODE, -1>), dim3((unsigned)nblk), dim3(512), 0,
-                         g_stream, *p, base, (const float *)src, (float *)dst);
+                         g_stream, *p, base, ntiles, (const float *)src, (float *)dst);
     else
       hipLaunchKernelGGL((k_c2c_mfma<NF, C, MODE, +1>), dim3((unsigned)nblk), dim3(512), 0,
-                         g_stream, *p, base, (const float *)src, (float *)dst);
+                         g_stream, *p, base, ntiles, (const float *)src, (float *)dst);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_error("pfk_launch_pass(mfma)", e); return -1; }
   }

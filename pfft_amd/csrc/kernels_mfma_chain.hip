@@ -260,7 +260,7 @@ k_mfma_tile(const pfk_pass P, const int64_t item0, const int64_t item_end, const
   constexpr int Q = NF / 16, R = Q / 16, KK = 4 / R;
   __shared__ cf ex[16 * NF];   // [n1][k2][line]
   __shared__ cf twl[NF];
-  stamp_begin(P);
+  stamp_begin(P, item0 + blockIdx.x);
   const int tid = threadIdx.x;
   twl[tid] = reinterpret_cast<const cf *>(P.tw)[tid];
   Coef<MODE, SIGN> K;
@@ -388,7 +388,7 @@ k_mfma_tile(const pfk_pass P, const int64_t item0, const int64_t item_end, const
   lds_barrier();   // twiddle table
   while (step(xa, xb) && step(xb, xa)) {
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - item);
 }
 
 // ---------------------------------------------------------------- line-major
@@ -436,7 +436,7 @@ k_mfma_line(const pfk_pass P, const int64_t item0, const int64_t item_end, const
   constexpr int SLOTS = NF + NF / 16;   // one line, one pad slot per 16 positions
   __shared__ cf twl[NF];
   __shared__ cf lx[4][SLOTS];           // per-wave transpose of a finished line
-  stamp_begin(P);
+  stamp_begin(P, item0 + blockIdx.x);
   const int tid = threadIdx.x;
   for (int i = tid; i < NF; i += 256) twl[i] = reinterpret_cast<const cf *>(P.tw)[i];
   Coef<MODE, SIGN> K;
@@ -566,7 +566,7 @@ k_mfma_line(const pfk_pass P, const int64_t item0, const int64_t item_end, const
   lds_barrier();   // twiddle table
   while (step(xa, xb) && step(xb, xa)) {
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - item);
 }
 
 template <typename K>

@@ -9,9 +9,10 @@ __global__ void __launch_bounds__(1024)
 k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const T *__restrict__ src,
         T *__restrict__ dst) {
   extern __shared__ unsigned char plane_smem[];
-  stamp_begin(P);
+  stamp_begin(P, blockIdx.x);
   bool tables = true;
-  for (int64_t id = blockIdx.x; id < nplanes; id += gridDim.x, tables = false) {
+  int64_t id = blockIdx.x;
+  for (; id < nplanes; id += gridDim.x, tables = false) {
     int64_t u = id, s = 0, d = 0;
     for (int i = 0; i < P.nb; ++i) {
       const int64_t k = u % P.bext[i];
@@ -21,7 +22,7 @@ k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const T *__re
     }
     plane_tile<T>(G, P.sign, src + 2 * s, dst + 2 * d, P.twm, P.pl.twm, tables, plane_smem);
   }
-  stamp_end(P);
+  stamp_end(P, nplanes - 1 - (id - gridDim.x));
 }
 
 static uint32_t recip(int64_t d) {

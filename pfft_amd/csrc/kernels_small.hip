@@ -10,22 +10,22 @@ namespace pfk {
 
 template <typename T, int NF>
 __global__ void __launch_bounds__(256)
-k_small(const pfk_pass P, const int64_t tile_base, const T *__restrict__ src,
-        T *__restrict__ dst) {
+k_small(const pfk_pass P, const int64_t tile_base, const int64_t ntiles,
+        const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
-  stamp_begin(P);
+  stamp_begin(P, tile_base + blockIdx.x);
   small_tile<T, NF>(P, tile_base + blockIdx.x, src, dst, smem_raw);
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - tile_base - blockIdx.x);
 }
 
 template <typename T, int NF, int KIND>
 __global__ void __launch_bounds__(256)
-k_small_real(const pfk_pass P, const int64_t tile_base, const T *__restrict__ src,
-             T *__restrict__ dst) {
+k_small_real(const pfk_pass P, const int64_t tile_base, const int64_t ntiles,
+             const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
-  stamp_begin(P);
+  stamp_begin(P, tile_base + blockIdx.x);
   small_split_real_tile<T, NF, KIND>(P, tile_base + blockIdx.x, src, dst, smem_raw);
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - tile_base - blockIdx.x);
 }
 
 // The length rule of small_covers for even r2c / c2r passes (without the
@@ -69,15 +69,15 @@ static int launch_small_nf(const pfk_pass *p, const void *src, void *dst) {
       const dim3 grid((unsigned)nblk), blk(small_threads(NF, F64, real));
       const size_t lds = small::lds_bytes(NF, F64, real);
       if (p->kind == PFK_C2C) {
-        hipLaunchKernelGGL((k_small<T, NF>), grid, blk, lds, g_stream, *p, base, (const T *)src,
-                           (T *)dst);
+        hipLaunchKernelGGL((k_small<T, NF>), grid, blk, lds, g_stream, *p, base, ntiles,
+                           (const T *)src, (T *)dst);
       } else if constexpr (split_real_length(NF, F64)) {
         if (p->kind == PFK_R2C)
           hipLaunchKernelGGL((k_small_real<T, NF, PFK_R2C>), grid, blk, lds, g_stream, *p, base,
-                             (const T *)src, (T *)dst);
+                             ntiles, (const T *)src, (T *)dst);
         else
           hipLaunchKernelGGL((k_small_real<T, NF, PFK_C2R>), grid, blk, lds, g_stream, *p, base,
-                             (const T *)src, (T *)dst);
+                             ntiles, (const T *)src, (T *)dst);
       } else {
         return 1;
       }

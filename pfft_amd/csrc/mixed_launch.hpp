@@ -12,14 +12,15 @@ __global__ void __launch_bounds__(512, 4)
 k_mixed(const pfk_pass P, const MixGeo G, const int64_t ntiles, const int64_t nlines,
         const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char mix_smem[];
-  stamp_begin(P);
+  stamp_begin(P, blockIdx.x);
   mix_table<T>(P, G, mix_smem);
   int odd = 0;
-  for (int64_t id = blockIdx.x; id < ntiles; id += gridDim.x, odd ^= 1) {
+  int64_t id = blockIdx.x;
+  for (; id < ntiles; id += gridDim.x, odd ^= 1) {
     const int64_t tile = P.xcd_remap ? xcd_remap(id, ntiles) : id;
     mixed_tile<T, KIND, BIG>(P, G, tile * G.C, nlines, odd, src, dst, mix_smem);
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - (id - gridDim.x));
 }
 
 // Launch with nt threads and `lds` bytes of LDS per workgroup.

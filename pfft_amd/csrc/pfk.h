@@ -149,9 +149,9 @@ typedef struct pfk_pass {
   int32_t mix_rad[PFK_MIX_MAXST];
   const void *twm;
   pfk_plane pl;
-  /* times of the pass (pfk_stamps; NULL: none): its first workgroup stores
-   * the clock to `stamp` when it starts, the last PFK_STAMP_ENDS workgroups
-   * store it to stamp_end[...] when they end */
+  /* times of the pass (pfk_stamps; NULL: none): the workgroup of its first
+   * work item stores the clock to `stamp` when it starts, those of its last
+   * PFK_STAMP_ENDS items store it to stamp_end[...] when they end */
   uint64_t *stamp, *stamp_end;
   /* element counts of the src/dst buffers, for host-side bounds checks */
   int64_t src_elems, dst_elems;

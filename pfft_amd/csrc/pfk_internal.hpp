@@ -25,17 +25,20 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Times of a pass (pfk_pass.stamp): at its start from workgroup 0, at its end
-// from the last workgroups of the grid, dispatched last and ending about last.
-// Every lane stores: a test of the thread index would keep it in a register to
-// the end, one more than the 128 that leave the 512-point complex128 kernels
-// 16 waves per CU (512^3 pair 2.28 -> 2.38 ms).
-__device__ __forceinline__ void stamp_begin(const pfk_pass &P) {
-  if (P.stamp && blockIdx.x == 0) *P.stamp = wall_clock64();
+// Times of a pass (pfk_pass.stamp): its start from the workgroup whose first
+// work item is item 0 of the pass, its end from the workgroups whose last item
+// is among the last PFK_STAMP_ENDS of the pass (`left` items follow it).  In a
+// walk b, b + grid, ... those are not the last workgroups of the grid: with
+// items left over after the full rounds, the low-numbered ones run them, and
+// the others end up to a round earlier.  Every lane stores: a test of the
+// thread index would keep it in a register to the end, one more than the 128
+// that leave the 512-point complex128 kernels 16 waves per CU (512^3 pair 2.28
+// -> 2.38 ms).
+__device__ __forceinline__ void stamp_begin(const pfk_pass &P, const int64_t first) {
+  if (P.stamp && first == 0) *P.stamp = wall_clock64();
 }
-__device__ __forceinline__ void stamp_end(const pfk_pass &P) {
-  const unsigned k = gridDim.x - 1 - blockIdx.x;
-  if (P.stamp_end && k < PFK_STAMP_ENDS) P.stamp_end[k] = wall_clock64();
+__device__ __forceinline__ void stamp_end(const pfk_pass &P, const int64_t left) {
+  if (P.stamp_end && left < PFK_STAMP_ENDS) P.stamp_end[left] = wall_clock64();
 }
 
 extern hipStream_t g_stream;

@@ -333,7 +333,7 @@ template <typename T, int NF, int C, int E, int SIGN, bool LM = false, bool TW =
 __global__ void __launch_bounds__(C *NF / E)
 k_c2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const int64_t ntiles,
            const T *__restrict__ src, T *__restrict__ dst) {
-  stamp_begin(P);
+  stamp_begin(P, item0 + blockIdx.x);
   constexpr int TT = NF / E;
   constexpr bool TWL = tw_in_lds<T>(lds_slots<NF, C, LM>(), NF, 0);
   __shared__ C2<T> lds[lds_slots<NF, C, LM>()];
@@ -438,7 +438,7 @@ k_c2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const 
   if constexpr (TWL) lds_barrier();
   while (step(va, vb) && step(vb, va)) {
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - item);
 }
 
 // ------------------------------------------------------------------ r2c
@@ -461,7 +461,7 @@ template <typename T, int NF, int C, int E, int SIGN, bool PL = false, bool LM =
 __global__ void __launch_bounds__(C *NF / E)
 k_r2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const int64_t ntiles,
            const T *__restrict__ src, T *__restrict__ dst) {
-  stamp_begin(P);
+  stamp_begin(P, item0 + blockIdx.x);
   constexpr int TT = NF / E;
   constexpr int H = NF;  // h = n/2
   constexpr bool TWL = tw_in_lds<T>(lds_slots<NF, C, LM>(), NF, NF);
@@ -556,7 +556,7 @@ k_r2c_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const 
   if constexpr (TWL) lds_barrier();
   while (step(va, vb) && step(vb, va)) {
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - item);
 }
 
 // ------------------------------------------------------------------ c2r
@@ -591,7 +591,7 @@ template <typename T, int NF, int C, int E, int SIGN, bool PL = false, bool LM =
 __global__ void __launch_bounds__(C *NF / E)
 k_c2r_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const int64_t ntiles,
            const T *__restrict__ src, T *__restrict__ dst) {
-  stamp_begin(P);
+  stamp_begin(P, item0 + blockIdx.x);
   constexpr int TT = NF / E;
   constexpr int H = NF;
   constexpr int SLOTS = LM ? lds_slots<NF, C, true>() : (NF + 1) * C;   // with the Nyquist bin
@@ -688,7 +688,7 @@ k_c2r_pow2(const pfk_pass P, const int64_t item0, const int64_t item_end, const 
   if constexpr (TWL) lds_barrier();
   while (step(va, ha, vb, hb) && step(vb, hb, va, ha)) {
   }
-  stamp_end(P);
+  stamp_end(P, ntiles - 1 - item);
 }
 
 // ------------------------------------------------------------------ dispatch
