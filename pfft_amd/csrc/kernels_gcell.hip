@@ -93,7 +93,7 @@ k_gc_fill(const GcDims d, const int64_t total, const T *__restrict__ src, T *__r
 // and of reduce's first part (local rows from their own box rows), a wave per
 // row: the row is decoded once per wave, and along the row the periodic source
 // is one subtraction, where the kernels above spend five integer divisions per
-// element.  For rows of at least a wave.
+// element.
 template <typename T, bool SS, bool SD, bool FILL>
 __device__ __forceinline__ void gc_rows(const GcDims &d, const T *__restrict__ src,
                                         T *__restrict__ dst) {
@@ -150,16 +150,29 @@ k_gc_own_rows(const GcDims d, const T *__restrict__ src, T *__restrict__ dst) {
   gc_rows<T, SS, SD, false>(d, src, dst);
 }
 
-// Single floats in rows of at least a wave, from 16 MiB on: the linear kernels'
-// divisions bound 4-byte elements (512^3, 4 ghost cells: exchange 515 -> 430 us,
-// reduce 495 -> 438).  With 8-byte elements they hide behind the accesses and the
+// Single floats in long rows, from 16 MiB on: the linear kernels' divisions
+// bound 4-byte elements (512^3, 4 ghost cells: exchange 515 -> 430 us, reduce
+// 495 -> 438).  With 8-byte elements they hide behind the accesses and the
 // longer contiguous runs of the linear kernels are faster (fill 378 against 409
 // us; float pairs, reduce 509 against 564), and small blocks lose 3 us to the
-// row's scalar arithmetic.
+// row's scalar arithmetic.  A wave spends its 16 loads a lane and its scalar
+// arithmetic on a row however short it is: by rows / linear, exchange 1.9 times
+// at 64 floats a row, 1.29 at 128, 1.06 at 192, 0.92-1.00 at 288, 0.8 from 512
+// on; reduce (16 loads wasted once, not twice) 1.3, 0.99, 0.89 and 0.85-0.95 at
+// the same widths (40 MiB blocks; 17 to 512 MiB cross 1 at the same widths).
 template <typename T>
-static bool gc_by_rows(const GcDims &d, int64_t nloc) {
-  return sizeof(T) == 4 && d.tuple == 1 && d.wloc >= 64 && nloc >= (int64_t)4 << 20;
+static bool gc_by_rows(const GcDims &d, int64_t nloc, uint32_t row, uint32_t min_row) {
+  return sizeof(T) == 4 && d.tuple == 1 && row >= min_row && nloc >= (int64_t)4 << 20;
 }
+#define GC_FILL_ROW 288
+#define GC_OWN_ROW 192
+
+// rows of whole 128-byte segments: a row kernel streams no others, their first
+// and last segments would be written in parts (fill at 800 MiB, rows of 508 and
+// 1108 floats streamed 735 and 759 us, not streamed 641 and 656; own rows of 1100
+// floats 822 streamed, 723 not, linear and streamed 722)
+template <typename T>
+static bool gc_whole_rows(uint32_t row) { return (size_t)row * sizeof(T) % 128 == 0; }
 
 // workgroups of a row kernel: a wave per row, at most 2^16 of them
 static int64_t gc_row_blocks(int64_t rows) {
@@ -348,17 +361,19 @@ int gc_event(void *const *ev, int k) {
     else hipLaunchKernelGGL((K<T, false, false>), grid_, blk_, 0, g_stream, __VA_ARGS__);              \
   } while (0)
 
-// Streaming: the user's array from blocks of 80 MiB on (50 MB blocks lost 4%),
-// the scratch copy where
-// it exceeds what the memory-side cache can hold (288 MiB, as the passes'):
-// exchange and reduce of 256^3 doubles with their two fills 368 -> 355 us,
-// 512^3 doubles 821 / 845 -> 797 / 823.
+// Streaming: the user's array from where it and the scratch copy together
+// exceed the memory-side cache, the scratch copy where it alone exceeds what
+// that can hold (288 MiB, as the passes').  Reduce of doubles, ordinary /
+// streamed user accesses: 100 MiB 81 / 86 us, 115 MiB 89 / 95, 128 MiB 118 /
+// 102, 200 MiB 196 / 143; exchange 85 / 86, 94 / 95, 105 / 103, 168 / 146.  Floats
+// take longer per byte and cross over later (exchange 128 MiB 140 / 143, 140
+// MiB 153 / 152).  512^3 doubles, everything streamed: 821 / 845 -> 797 / 823.
 struct GcStreams {
   bool user, scratch;
 };
 static GcStreams gc_streams(int64_t nloc, size_t esz) {
   const double bytes = (double)nloc * (double)esz;
-  return GcStreams{bytes >= 80.0 * 1048576, bytes > 288.0 * 1048576};
+  return GcStreams{bytes >= (esz == 4 ? 140.0 : 128.0) * 1048576, bytes > 288.0 * 1048576};
 }
 
 template <typename T>
@@ -368,14 +383,16 @@ int gc_exchange(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   if (gc_dims(g, &d, &L, &G)) return 1;
   if (gc_event(ev, 0)) return 1;
   // block copy: the compact kernel with nothing to zero
-  const GcStreams st = gc_streams(L, sizeof(T));
+  GcStreams st = gc_streams(L, sizeof(T));
+  const bool rows = gc_by_rows<T>(d, L, d.wbox, GC_FILL_ROW);
+  if (rows && st.scratch && !gc_whole_rows<T>(d.wbox)) st = GcStreams{false, false};
   GC_LAUNCH(k_gc_compact, T, st.user, st.scratch, (L + GC_CH - 1) / GC_CH, L, L, (const T *)data,
             scratch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_gc_exchange copy", e); return 1; }
   if (gc_event(ev, 1)) return 1;
   const int64_t nb = (G + GC_CH - 1) / GC_CH;
-  if (gc_by_rows<T>(d, L))
+  if (rows)
     GC_LAUNCH(k_gc_fill_rows, T, st.scratch, st.user, gc_row_blocks(g->ngc[0] * g->ngc[1]), d,
               (const T *)scratch, data);
   else
@@ -406,7 +423,7 @@ int gc_reduce(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   sh.c2 = I[0] * I[1] * E[2] * g->tuple;
   if (gc_event(ev, 0)) return 1;
   const GcStreams st = gc_streams(L, sizeof(T));
-  if (gc_by_rows<T>(d, L))
+  if (gc_by_rows<T>(d, L, d.wloc, GC_OWN_ROW) && (!st.scratch || gc_whole_rows<T>(d.wloc)))
     GC_LAUNCH(k_gc_own_rows, T, st.user, st.scratch, gc_row_blocks(g->n[0] * g->n[1]), d,
               (const T *)data, scratch);
   else
