@@ -361,19 +361,20 @@ int gc_event(void *const *ev, int k) {
     else hipLaunchKernelGGL((K<T, false, false>), grid_, blk_, 0, g_stream, __VA_ARGS__);              \
   } while (0)
 
-// Streaming: the user's array from where it and the scratch copy together
-// exceed the memory-side cache, the scratch copy where it alone exceeds what
-// that can hold (288 MiB, as the passes').  Reduce of doubles, ordinary /
-// streamed user accesses: 100 MiB 81 / 86 us, 115 MiB 89 / 95, 128 MiB 118 /
-// 102, 200 MiB 196 / 143; exchange 85 / 86, 94 / 95, 105 / 103, 168 / 146.  Floats
-// take longer per byte and cross over later (exchange 128 MiB 140 / 143, 140
-// MiB 153 / 152).  512^3 doubles, everything streamed: 821 / 845 -> 797 / 823.
+// Streaming: the user's array from where its box and the scratch copy together
+// exceed the 256 MiB memory-side cache, the scratch copy where it alone exceeds
+// what that can hold (288 MiB, as the passes').  User's array streamed /
+// ordinary by the MiB of box and copy, doubles, 1 to 8 ghost cells, rows of 120
+// and 256: reduce 236 MiB 1.07-1.10, 252 0.95-1.10, 264 0.89-0.95, 320
+// 0.76-0.85; exchange 1.02, 1.01, 0.96-1.01, 0.87-0.90.  Floats take longer per
+// byte and cross later: 264 0.98-1.03, 272 0.95-1.01.  512^3 doubles, everything
+// streamed: 821 / 845 -> 797 / 823 us.
 struct GcStreams {
   bool user, scratch;
 };
-static GcStreams gc_streams(int64_t nloc, size_t esz) {
-  const double bytes = (double)nloc * (double)esz;
-  return GcStreams{bytes >= (esz == 4 ? 140.0 : 128.0) * 1048576, bytes > 288.0 * 1048576};
+static GcStreams gc_streams(int64_t nloc, int64_t nbox, size_t esz) {
+  const double mib = (double)esz / 1048576, both = mib * (double)(nloc + nbox);
+  return GcStreams{both >= (esz == 4 ? 272.0 : 264.0), mib * (double)nloc > 288.0};
 }
 
 template <typename T>
@@ -383,7 +384,7 @@ int gc_exchange(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   if (gc_dims(g, &d, &L, &G)) return 1;
   if (gc_event(ev, 0)) return 1;
   // block copy: the compact kernel with nothing to zero
-  GcStreams st = gc_streams(L, sizeof(T));
+  GcStreams st = gc_streams(L, G, sizeof(T));
   const bool rows = gc_by_rows<T>(d, L, d.wbox, GC_FILL_ROW);
   if (rows && st.scratch && !gc_whole_rows<T>(d.wbox)) st = GcStreams{false, false};
   GC_LAUNCH(k_gc_compact, T, st.user, st.scratch, (L + GC_CH - 1) / GC_CH, L, L, (const T *)data,
@@ -422,7 +423,7 @@ int gc_reduce(const pfk_gc *g, T *data, T *scratch, void *const *ev) {
   sh.c1 = I[0] * E[1] * g->n[2] * g->tuple;
   sh.c2 = I[0] * I[1] * E[2] * g->tuple;
   if (gc_event(ev, 0)) return 1;
-  const GcStreams st = gc_streams(L, sizeof(T));
+  const GcStreams st = gc_streams(L, G, sizeof(T));
   if (gc_by_rows<T>(d, L, d.wloc, GC_OWN_ROW) && (!st.scratch || gc_whole_rows<T>(d.wloc)))
     GC_LAUNCH(k_gc_own_rows, T, st.user, st.scratch, gc_row_blocks(g->n[0] * g->n[1]), d,
               (const T *)data, scratch);

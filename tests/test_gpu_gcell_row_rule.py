@@ -44,7 +44,7 @@ def test_floats_no_slower_than_doubles(n):
     ([160, 160, 191], [1, 0, 1], [0, 1, 0]), ([160, 160, 192], [1, 0, 1], [0, 1, 2]),
     ([130, 128, 287], [1, 0, 0], [0, 1, 0]), ([130, 128, 287], [1, 0, 1], [0, 1, 0]),
     ([130, 128, 288], [0, 2, 0], [1, 0, 300]), ([700, 220, 30], [1, 1, 130], [0, 0, 140]),
-    # user's array streamed (140 MiB and more), by rows and linear
+    # user's array streamed, its copy not (272 MiB of both and more), by rows and linear
     ([200, 400, 500], [1, 0, 6], [0, 1, 6]), ([400, 990, 100], [1, 0, 6], [0, 1, 6]),
     # above 288 MiB: whole segments, ragged rows, ragged boxes
     ([300, 500, 512], [1, 0, 16], [0, 1, 16]), ([300, 500, 512], [1, 0, 1], [0, 1, 1]),
