@@ -224,11 +224,14 @@ static int batch_capture_forked(pfk_batch *b) {
   return err;
 }
 
+static bool batch_short(const pfk_pass *p) {
+  return !g_generic_only && p->variant != 1 && p->kind == PFK_C2C && small_covers(p) &&
+         batch_small_length((int)p->nf, p->prec == PFK_F64);
+}
+
 static int task_class(const pfk_task *t) {
   if (t->pass.pl.n) return PFK_PLANE_CLASS + plane_threads(&t->pass) / 64;
-  if (!g_generic_only && t->pass.variant != 1 && t->pass.kind == PFK_C2C &&
-      small_covers(&t->pass) && batch_small_length((int)t->pass.nf, t->pass.prec == PFK_F64))
-    return (int)t->pass.nf;
+  if (batch_short(&t->pass)) return (int)t->pass.nf;
   return 0;
 }
 
@@ -342,6 +345,8 @@ static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task
   }
   return 0;
 }
+
+extern "C" int pfk_batch_short(const pfk_pass *p) { return batch_short(p) ? 1 : 0; }
 
 extern "C" pfk_batch *pfk_batch_create(pfk_task *tasks, int ntasks, int use_graph) {
   if (pfk_init() || ntasks <= 0) return nullptr;

@@ -365,6 +365,9 @@ int  pfk_pass_kernels(const pfk_pass *p);
  * modulation or weights): the instantiations without masks run it */
 int  pfk_pass_plain(const pfk_pass *p);
 
+/* 1 if a batch runs the pass with the short-length kernel. */
+int  pfk_batch_short(const pfk_pass *p);
+
 /* LDS bytes of a plane pass (pl.n set), 0 if it has no kernel. */
 size_t pfk_plane_covers(const pfk_pass *p);
 

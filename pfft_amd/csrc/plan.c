@@ -1110,11 +1110,29 @@ static int64_t batch_planes(const pa_plan *const *plans, int count) {
 }
 #define PA_BATCH_PLANES 1024
 
+/* Whether the plan runs fused in a batch of `planes` planes.  Every plane costs
+ * a workgroup the same setup (its task, its offsets, the twiddle tables, a
+ * barrier a stage), however small it is, where the short-length passes put many
+ * lines into a workgroup: small planes with such passes on both sides pay only
+ * while the batch is small, up to about 96 planes a point.  Planes / three
+ * passes, complex128 and complex64: 4x4, 1104 planes 0.98 and 0.98, 12800 1.12
+ * and 1.06, 40000 1.42 and 1.36; 8x8, 4096 0.97 and 0.94, 12800 1.08 and 0.99,
+ * 25600 1.22 and 1.05; 12x16, 12800 1.00 and 0.96, 25600 1.08 and 1.05; 16x16,
+ * 25600 1.00 and 1.10; 16x24, 25600 0.94 and 0.85; 24x24 1.03 and 0.82; 5x7,
+ * without a short-length pass, 5000 0.79 and 0.84. */
+static int batch_fuses(const pa_plan *p, int64_t planes) {
+  if (!p->nfused || planes < PA_BATCH_PLANES) return 0;
+  const pfk_pass *col = &p->pass[p->pass_of[1]], *row = &p->pass[p->pass_of[2]];
+  const int64_t points = p->n[1] * p->n[2];
+  return points >= 320 || planes <= 96 * points || !pfk_batch_short(col) ||
+         !pfk_batch_short(row);
+}
+
 static pfk_batch *batch_build(const pa_plan *const *plans, int count) {
   int maxp = 0, ntasks = 0;
-  const int fuse = batch_planes(plans, count) >= PA_BATCH_PLANES;
+  const int64_t planes = batch_planes(plans, count);
   for (int i = 0; i < count; i++) {
-    const int n = prog_n(plans[i], fuse && plans[i]->nfused);
+    const int n = prog_n(plans[i], batch_fuses(plans[i], planes));
     if (n > maxp) maxp = n;
     ntasks += n;
   }
@@ -1125,7 +1143,7 @@ static pfk_batch *batch_build(const pa_plan *const *plans, int count) {
   for (int lev = 0; lev < maxp; lev++)
     for (int i = 0; i < count; i++) {
       const pa_plan *p = plans[i];
-      const int fused = fuse && p->nfused;
+      const int fused = batch_fuses(p, planes);
       if (lev >= prog_n(p, fused)) continue;
       void *bufs[4] = {p->in, p->out, p->scratch[0], p->scratch[1]};
       tasks[k].pass = *prog_pass(p, fused, lev);
@@ -1238,14 +1256,14 @@ int pa_plans_execute_batch_noalloc(const pa_plan *const *plans, int count) {
   /* level order (every plan's pass 0, then every pass 1, ...), each task
    * depending on the previous pass of its plan: within the block of level
    * lev-1 the plans with at least lev passes appear in plan order */
-  const int fuse = batch_planes(plans, count) >= PA_BATCH_PLANES;
+  const int64_t planes = batch_planes(plans, count);
   int k = 0, prev_start = 0;
   for (int lev = 0; lev < maxp; lev++) {
     const int cur_start = k;
     int a = prev_start;
     for (int i = 0; i < count; i++) {
       const pa_plan *p = plans[i];
-      const int fused = fuse && p->nfused;
+      const int fused = batch_fuses(p, planes);
       const int in_prev = lev > 0 && prog_n(p, fused) > lev - 1;
       if (lev < prog_n(p, fused)) {
         void *bufs[4] = {p->in, p->out, p->scratch[0], p->scratch[1]};
