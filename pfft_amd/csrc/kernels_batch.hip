@@ -24,6 +24,11 @@
 
 namespace pfk {
 
+// Every workgroup searches the work-list and a no-alloc batch uploads it on each
+// call: with the geometry of a plane in every task (968 bytes) such batches of 60
+// to 400 small plans took 3-10 % longer than at 560 bytes; 608 are level with it.
+static_assert(sizeof(pfk_task) <= 608, "size of a work-list entry");
+
 // task of work-list item g within tasks [t0, t1)
 __device__ __forceinline__ int find_task(const pfk_task *__restrict__ tasks, int t0, int t1,
                                          int64_t g) {
@@ -70,16 +75,19 @@ k_batch_small(const pfk_task *__restrict__ tasks, const int t0, const int t1,
   }
 }
 
-// plane passes: an item is a plane
+// plane passes: an item is a plane.  The geometries are a parameter, not a
+// pointer in the task: only then are they known to stay as they are while the
+// planes are stored, and read once (64 transforms of 64^3 complex128 294 us, 373
+// through a pointer).
 template <typename T>
 __global__ void __launch_bounds__(1024)
 k_batch_plane(const pfk_task *__restrict__ tasks, const int t0, const int t1,
-              const int64_t item0, const int64_t item1) {
+              const int64_t item0, const int64_t item1, const PlaneGeo *__restrict__ geo) {
   extern __shared__ unsigned char smem_raw[];
   for (int64_t g = item0 + blockIdx.x; g < item1; g += gridDim.x) {
     const pfk_task &tk = tasks[find_task(tasks, t0, t1, g)];
     const pfk_pass &P = tk.pass;
-    const PlaneGeo &G = *reinterpret_cast<const PlaneGeo *>(tk.plane);
+    const PlaneGeo &G = geo[tk.geo];
     int64_t u = g - tk.first_item, s = 0, d = 0;
     for (int i = 0; i < P.nb; ++i) {
       const int64_t k = u % P.bext[i];
@@ -87,11 +95,9 @@ k_batch_plane(const pfk_task *__restrict__ tasks, const int t0, const int t1,
       s += k * P.bsin[i];
       d += k * P.bsout[i];
     }
-    plane_tile<T>(G, P.sign, (const T *)tk.src + 2 * s, (T *)tk.dst + 2 * d, P.twm, P.pl.twm, true,
-                  smem_raw);
+    plane_tile<T>(G, P.sign, (const T *)tk.src + 2 * s, (T *)tk.dst + 2 * d, P.twm, G.twc, true, smem_raw);
   }
 }
-static_assert(sizeof(PlaneGeo) <= sizeof(pfk_task::plane), "plane geometry in a task");
 
 // short lengths the batch runs with the short-length kernel: those whose
 // workgroups have 4 waves (the batch launches 256 threads), odd lengths
@@ -146,9 +152,11 @@ typedef struct {
   size_t lds;
 } batch_group;
 
+// The device work-list: the tasks and behind them the geometry of the plane
+// passes among them (apart, for the tasks are searched and most have none).
 struct pfk_batch {
   pfk_task *d_tasks;
-  int ntasks;
+  int ntasks, nplanes;
   int ngroups;
   batch_group groups[PFK_MAX_GROUPS];
   int use_graph;
@@ -163,7 +171,9 @@ static int launch_group(const pfk_batch *b, const batch_group *g, hipStream_t s)
   const pfk_task *tasks = b->d_tasks;
   int t0 = g->t0, t1 = g->t1;
   int64_t i0 = g->i0, i1 = g->i1;
-  void *args[] = {(void *)&tasks, (void *)&t0, (void *)&t1, (void *)&i0, (void *)&i1};
+  const PlaneGeo *geo = reinterpret_cast<const PlaneGeo *>(tasks + b->ntasks);   // plane kernel
+  void *args[] = {(void *)&tasks, (void *)&t0, (void *)&t1,
+                  (void *)&i0, (void *)&i1, (void *)&geo};
   hipError_t e = hipLaunchKernel(g->kernel, dim3(grid), dim3(g->threads), args, g->lds, s);
   if (e == hipSuccess) e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_batch launch", e); return 1; }
@@ -230,7 +240,7 @@ static bool batch_short(const pfk_pass *p) {
 }
 
 static int task_class(const pfk_task *t) {
-  if (t->pass.pl.n) return PFK_PLANE_CLASS + plane_threads(&t->pass) / 64;
+  if (t->pass.pl) return PFK_PLANE_CLASS + plane_threads(&t->pass) / 64;
   if (batch_short(&t->pass)) return (int)t->pass.nf;
   return 0;
 }
@@ -255,8 +265,10 @@ static int sort_level(pfk_task *a, int n, pfk_task *tmp) {
  * task.dep marks the previous pass of the same plan, so a task whose dep
  * lies in the current level starts a new level.  The array is reordered
  * (by kernel within each level, through `tmp`, room for ntasks) and its
- * tiling fields filled. */
-static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task *tmp) {
+ * tiling fields filled; the geometries of its b->nplanes plane passes go to
+ * `geo`. */
+static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task *tmp,
+                             PlaneGeo *geo) {
   const int prec = tasks[0].pass.prec;
   int lev_start[PFK_MAXSTAGES + 1], nlev = 0;
   lev_start[0] = 0;
@@ -272,6 +284,7 @@ static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task
   }
   lev_start[++nlev] = ntasks;
   b->ntasks = ntasks;
+  b->nplanes = 0;
   b->ngroups = 0;
   int dev = 0, ncu = 0;
   (void)hipGetDevice(&dev);
@@ -299,11 +312,11 @@ static int batch_plan_levels(pfk_batch *b, pfk_task *tasks, int ntasks, pfk_task
         size_t ld;
         int64_t nt;
         if (cls > PFK_PLANE_CLASS) {
-          if (plane_geo(&t->pass, 64 * (cls - PFK_PLANE_CLASS),
-                        reinterpret_cast<PlaneGeo *>(t->plane), &ld)) {
+          if (plane_geo(&t->pass, 64 * (cls - PFK_PLANE_CLASS), geo + b->nplanes, &ld)) {
             set_error_msg("pfk_batch: bad plane pass");
             return 1;
           }
+          t->geo = b->nplanes++;
           nt = 1;
           for (int k = 0; k < t->pass.nb; k++) nt *= t->pass.bext[k];
         } else if (cls) {
@@ -354,12 +367,17 @@ extern "C" pfk_batch *pfk_batch_create(pfk_task *tasks, int ntasks, int use_grap
   if (!b) return nullptr;
   b->use_graph = use_graph;
   pfk_task *tmp = (pfk_task *)malloc(sizeof(pfk_task) * (size_t)ntasks);
-  const int bad = !tmp || batch_plan_levels(b, tasks, ntasks, tmp);
+  PlaneGeo *geo = (PlaneGeo *)malloc(sizeof(PlaneGeo) * (size_t)ntasks);
+  const int bad = !tmp || !geo || batch_plan_levels(b, tasks, ntasks, tmp, geo);
   free(tmp);
-  if (bad) { free(b); return nullptr; }
-  hipError_t e = hipMalloc(&b->d_tasks, sizeof(pfk_task) * ntasks);
-  if (e == hipSuccess)
-    e = hipMemcpy(b->d_tasks, tasks, sizeof(pfk_task) * ntasks, hipMemcpyHostToDevice);
+  if (bad) { free(geo); free(b); return nullptr; }
+  const size_t task_bytes = sizeof(pfk_task) * (size_t)ntasks;
+  const size_t geo_bytes = sizeof(PlaneGeo) * (size_t)b->nplanes;
+  hipError_t e = hipMalloc(&b->d_tasks, task_bytes + geo_bytes);
+  if (e == hipSuccess) e = hipMemcpy(b->d_tasks, tasks, task_bytes, hipMemcpyHostToDevice);
+  if (e == hipSuccess && geo_bytes)
+    e = hipMemcpy(b->d_tasks + ntasks, geo, geo_bytes, hipMemcpyHostToDevice);
+  free(geo);
   if (e != hipSuccess) { set_error("pfk_batch_create", e); pfk_batch_destroy(b); return nullptr; }
   if (use_graph) {
     e = hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal);
@@ -380,11 +398,13 @@ extern "C" pfk_batch *pfk_batch_create(pfk_task *tasks, int ntasks, int use_grap
 // address hipGetSymbolAddress returns for the current device, never the
 // symbol itself.
 #define PFK_NOALLOC_TASKS 2048
-static __device__ __align__(256) unsigned char scratch[sizeof(pfk_task) * PFK_NOALLOC_TASKS];
+static __device__ __align__(256) unsigned char
+    scratch[(sizeof(pfk_task) + sizeof(PlaneGeo)) * PFK_NOALLOC_TASKS];
 #define PFK_MAX_DEVICES 64
 static void *g_scratch_ptr[PFK_MAX_DEVICES];
 static pfk_batch g_noalloc_batch;                 // group table (host memory)
 static pfk_task g_noalloc_tmp[PFK_NOALLOC_TASKS];  // sort buffer (host memory)
+static PlaneGeo g_noalloc_geo[PFK_NOALLOC_TASKS];  // plane geometries (host memory)
 
 extern "C" int pfk_batch_run_noalloc(pfk_task *tasks, int ntasks) {
   if (pfk_init()) return 1;
@@ -408,10 +428,13 @@ extern "C" int pfk_batch_run_noalloc(pfk_task *tasks, int ntasks) {
   }
   pfk_batch *b = &g_noalloc_batch;
   b->use_graph = 0;
-  if (batch_plan_levels(b, tasks, ntasks, g_noalloc_tmp)) return 1;
+  if (batch_plan_levels(b, tasks, ntasks, g_noalloc_tmp, g_noalloc_geo)) return 1;
   b->d_tasks = (pfk_task *)g_scratch_ptr[dev];
   e = hipMemcpyAsync(b->d_tasks, tasks, sizeof(pfk_task) * (size_t)ntasks, hipMemcpyHostToDevice,
                      g_stream);
+  if (e == hipSuccess && b->nplanes)
+    e = hipMemcpyAsync(b->d_tasks + ntasks, g_noalloc_geo, sizeof(PlaneGeo) * (size_t)b->nplanes,
+                       hipMemcpyHostToDevice, g_stream);
   if (e != hipSuccess) { set_error("pfk_batch_run_noalloc: work-list upload", e); return 1; }
   if (batch_launch(b)) return 1;
   e = hipStreamSynchronize(g_stream);

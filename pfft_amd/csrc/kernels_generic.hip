@@ -893,7 +893,7 @@ int pfk_pass_check(const pfk_pass *p) {
 
 int pfk_launch_pass(const pfk_pass *p, const void *src, void *dst) {
   if (pfk_init()) return 1;
-  if (p->pl.n) return launch_plane(p, src, dst);
+  if (p->pl) return launch_plane(p, src, dst);
   if (p->kind == PFK_R2R && p->r2r_path) {
     const int f = g_generic_only ? 1 : launch_mixed(p, src, dst);
     return f > 0 ? r2r_real_path(p, src, dst) : f < 0;

@@ -20,7 +20,7 @@ k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const T *__re
       s += k * P.bsin[i];
       d += k * P.bsout[i];
     }
-    plane_tile<T>(G, P.sign, src + 2 * s, dst + 2 * d, P.twm, P.pl.twm, tables, plane_smem);
+    plane_tile<T>(G, P.sign, src + 2 * s, dst + 2 * d, P.twm, G.twc, tables, plane_smem);
   }
   stamp_end(P, nplanes - 1 - (id - gridDim.x));
 }
@@ -30,7 +30,7 @@ static uint32_t recip(int64_t d) {
 }
 
 static size_t plane_lds(const pfk_pass *p, PlaneGeo *g) {
-  g->n1 = (int)p->pl.n;
+  g->n1 = (int)p->pl->n;
   g->n2 = (int)p->nf;
   g->pitch = g->n2 + ((g->n2 - 1) >> 4) + 1;
   int L = 1;
@@ -40,9 +40,9 @@ static size_t plane_lds(const pfk_pass *p, PlaneGeo *g) {
     L *= p->mix_rad[s];
   }
   L = 1;
-  for (int s = 0; s < p->pl.mix_n; s++) {
-    if (s) g->ntw2 += (p->pl.mix_rad[s] - 1) * L;
-    L *= p->pl.mix_rad[s];
+  for (int s = 0; s < p->pl->mix_n; s++) {
+    if (s) g->ntw2 += (p->pl->mix_rad[s] - 1) * L;
+    L *= p->pl->mix_rad[s];
   }
   return (size_t)(g->ntw1 + g->ntw2 + g->n1 * g->pitch) * (p->prec == PFK_F64 ? 16 : 8);
 }
@@ -54,18 +54,19 @@ int plane_threads(const pfk_pass *p) {
 }
 
 int plane_geo(const pfk_pass *p, int nt, PlaneGeo *g, size_t *lds) {
-  if (p->pl.n < 2 || p->nf < 2 || p->pl.n > 1024 || p->nf > 1024 || !p->twm || !p->pl.twm ||
-      p->mix_n < 1 || p->pl.mix_n < 1 || p->mix_n + p->pl.mix_n > PFK_PLANE_MAXST)
+  if (p->pl->n < 2 || p->nf < 2 || p->pl->n > 1024 || p->nf > 1024 || !p->twm || !p->pl->twm ||
+      p->mix_n < 1 || p->pl->mix_n < 1 || p->mix_n + p->pl->mix_n > PFK_PLANE_MAXST)
     return 1;
   *lds = plane_lds(p, g);
   // Larger planes leave a CU one workgroup, whose load, stages and store follow
   // one another (384 uneven complex64 transforms: 1093 us at 110 KiB, 1118 at
   // 150, 1210 at 72, 1430 without planes).
   if (*lds > 110 * 1024) return 1;
-  g->nst = p->mix_n + p->pl.mix_n;
+  g->nst = p->mix_n + p->pl->mix_n;
   g->nrow = p->mix_n;
-  g->s1 = p->pl.sin;
-  g->d1 = p->pl.sout;
+  g->s1 = p->pl->sin;
+  g->d1 = p->pl->sout;
+  g->twc = p->pl->twm;
   g->keep_ld = (p->cache & PFK_KEEP_SRC) != 0;
   g->keep_st = (p->cache & PFK_KEEP_DST) != 0;
   int L = 1, tw = 0;
@@ -73,7 +74,7 @@ int plane_geo(const pfk_pass *p, int nt, PlaneGeo *g, size_t *lds) {
     const bool col = s >= p->mix_n;
     if (s == p->mix_n) { L = 1; tw = g->ntw1; }
     const int n = col ? g->n1 : g->n2, lines = col ? g->n2 : g->n1;
-    const int R = col ? p->pl.mix_rad[s - p->mix_n] : p->mix_rad[s];
+    const int R = col ? p->pl->mix_rad[s - p->mix_n] : p->mix_rad[s];
     if (R > 16) return 1;
     PlaneStage *t = &g->st[s];
     t->R = R;

@@ -80,9 +80,9 @@ typedef struct pfk_mod {
  * (contiguous on both sides, every position present) and n lines of it, sin /
  * sout apart, are transformed together along both dimensions. */
 typedef struct pfk_plane {
-  int64_t n, sin, sout;   /* n 0: no plane */
-  int32_t mix_n;
-  int32_t mix_rad[PFK_MIX_MAXST];
+  int64_t n, sin, sout;
+  int16_t mix_n;
+  int16_t mix_rad[PFK_MIX_MAXST];
   const void *twm;        /* stage table of length n (pfk_pass.twm) */
 } pfk_plane;
 
@@ -145,10 +145,10 @@ typedef struct pfk_pass {
    * and the forward twiddles in stage order: for stage s > 0 with L the
    * product of the earlier radices, W_(L R)^(r k) at [(r-1) L + k], r in
    * [1, R), k in [0, L), and behind them, for a radix above 16, W_R^m, m < R */
-  int32_t mix_n;
-  int32_t mix_rad[PFK_MIX_MAXST];
+  int16_t mix_n;
+  int16_t mix_rad[PFK_MIX_MAXST];
   const void *twm;
-  pfk_plane pl;
+  const pfk_plane *pl;   /* host memory; NULL: no plane */
   /* times of the pass (pfk_stamps; NULL: none): the workgroup of its first
    * work item stores the clock to `stamp` when it starts, those of its last
    * PFK_STAMP_ENDS items store it to stamp_end[...] when they end */
@@ -187,17 +187,18 @@ static inline int pfk_factorize(int64_t nf, int32_t *radix) {
  * largest that is 2 mod 4 (its stores to LDS then meet no bank twice), the
  * others follow in descending order.  Returns the stage count, 0 if there are
  * more than PFK_MIX_MAXST. */
-static inline int pfk_mix_search(int64_t m, int maxr, int left, int32_t *out) {
+static inline int pfk_mix_search(int64_t m, int maxr, int left, int16_t *out) {
   if (m == 1) return 1;
   if (left == 0) return 0;
   for (int r = maxr; r >= 2; r--)
     if (m % r == 0) {
-      out[0] = r;
+      out[0] = (int16_t)r;
       if (pfk_mix_search(m / r, r, left - 1, out + 1)) return 1;
     }
   return 0;
 }
-static inline int pfk_mix_factorize(int64_t nf, int32_t *rad) {
+static inline int pfk_mix_factorize(int64_t nf, int16_t *rad) {
+  if (nf > 4096) return 0;   /* PFK_MAXLINE */
   int big = 0;
   int64_t rest = 1, m = nf;
   for (int64_t q = 2; m > 1; q++) {   /* primes in ascending order */
@@ -207,7 +208,7 @@ static inline int pfk_mix_factorize(int64_t nf, int32_t *rad) {
         rest *= q;
       } else {
         if (big == PFK_MIX_MAXST) return 0;
-        rad[big++] = (int32_t)q;
+        rad[big++] = (int16_t)q;
       }
     }
   }
@@ -215,13 +216,13 @@ static inline int pfk_mix_factorize(int64_t nf, int32_t *rad) {
   for (int n = 1; rest > 1 && n <= PFK_MIX_MAXST - big; n++)
     for (int maxr = 2; maxr <= 16; maxr++)
       if (pfk_mix_search(rest, maxr, n, rad + big)) {
-        int32_t *r = rad + big;
+        int16_t *r = rad + big;
         int k = 0, f = 0;
         for (int64_t m = rest; m > 1; k++) m /= r[k];
         while (f < k && r[f] % 2 == 0) f++;
         if (f == k) for (f = 0; f < k && r[f] % 4 != 2; f++) { }
         if (f < k) {
-          const int32_t r0 = r[f];
+          const int16_t r0 = r[f];
           for (; f > 0; f--) r[f] = r[f - 1];
           r[0] = r0;
         }
@@ -259,8 +260,7 @@ typedef struct pfk_task {
   int64_t ntiles;         /* filled by pfk_batch_create */
   int64_t first_item;     /* filled by pfk_batch_create */
   int32_t dep;
-  int32_t pad;
-  int64_t plane[36];      /* plane passes: their launch geometry, filled by pfk_batch_create */
+  int32_t geo;            /* plane passes: index of their geometry, filled by pfk_batch_create */
 } pfk_task;
 
 /* Batched execution of many passes: tasks grouped by pass level, one
@@ -368,7 +368,7 @@ int  pfk_pass_plain(const pfk_pass *p);
 /* 1 if a batch runs the pass with the short-length kernel. */
 int  pfk_batch_short(const pfk_pass *p);
 
-/* LDS bytes of a plane pass (pl.n set), 0 if it has no kernel. */
+/* LDS bytes of a plane pass (pl set), 0 if it has no kernel. */
 size_t pfk_plane_covers(const pfk_pass *p);
 
 /* Timing helpers on the library stream (HIP events). */

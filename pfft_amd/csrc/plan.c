@@ -73,7 +73,9 @@ struct pa_plan {
   /* The passes as executed where two dimensions share one (fuse_planes): pass
    * fused[i] does logical dimensions fdim[i][0] and, for a plane, fdim[i][1] */
   int nfused;
+  pfk_plane plane;               /* of the fused pass that has one */
   int fused_alone;               /* also where the plan runs by itself */
+  int batch_short;               /* in a batch both sides of a plane have short-length passes */
   pfk_pass fused[2];
   int fsrc[2], fdst[2], fdim[2][2];
   int pass_of[PA_MAXRNK];        /* pass of a logical dimension */
@@ -426,12 +428,13 @@ static void fuse_planes(pa_plan *p, const arrgeo *geo, const int *ord) {
       q->bext[0] = p->n[0];
       q->bsin[0] = ss[0];
       q->bsout[0] = sd[0];
-      q->pl.n = p->n[1];
-      q->pl.sin = ss[1];
-      q->pl.sout = sd[1];
-      q->pl.mix_n = col->mix_n;
-      memcpy(q->pl.mix_rad, col->mix_rad, sizeof q->pl.mix_rad);
-      q->pl.twm = col->twm;
+      p->plane.n = p->n[1];
+      p->plane.sin = ss[1];
+      p->plane.sout = sd[1];
+      p->plane.mix_n = col->mix_n;
+      memcpy(p->plane.mix_rad, col->mix_rad, sizeof p->plane.mix_rad);
+      p->plane.twm = col->twm;
+      q->pl = &p->plane;
       if ((p->n[0] - 1) * ss[0] + (p->n[1] - 1) * ss[1] + p->n[2] > q->src_elems ||
           (p->n[0] - 1) * sd[0] + (p->n[1] - 1) * sd[1] + p->n[2] > q->dst_elems ||
           !pfk_plane_covers(q))
@@ -915,6 +918,9 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
     }
   fuse_planes(p, geo, ord);
   tune_plan(p);
+  if (p->nfused)
+    p->batch_short = pfk_batch_short(&p->pass[p->pass_of[1]]) &&
+                     pfk_batch_short(&p->pass[p->pass_of[2]]);
   return p;
 fail:
   free_plan_memory(p);
@@ -980,6 +986,7 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
     const int k = adjoint ? np - 1 - i : i;
     const pfk_pass *fw = prog_pass(p, fused, k);
     pfk_pass a = *fw;
+    pfk_plane pl;
     a.stamp = stamps ? stamps + i : NULL;
     a.stamp_end = stamps && i == np - 1 ? stamps + PFK_STAMPS - PFK_STAMP_ENDS : NULL;
     if (!adjoint) {
@@ -992,12 +999,16 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
       a.sin = fw->sout; a.sout = fw->sin;
       a.tsin = fw->tsout; a.tsout = fw->tsin;
       for (int b = 0; b < a.nb; b++) { a.bsin[b] = fw->bsout[b]; a.bsout[b] = fw->bsin[b]; }
-      a.pl.sin = fw->pl.sout; a.pl.sout = fw->pl.sin;
+      if (fw->pl) {
+        pl = *fw->pl;
+        pl.sin = fw->pl->sout; pl.sout = fw->pl->sin;
+        a.pl = &pl;
+      }
       a.src_elems = fw->dst_elems; a.dst_elems = fw->src_elems;
       if (fw->kind == PFK_R2C) { a.kind = PFK_C2R; a.hw = 1; }
       else if (fw->kind == PFK_C2R) { a.kind = PFK_R2C; a.hw = 2; }
       if (!fused) { a.tw = p->tw_adj[k]; a.rtw = p->rtw_adj[k]; }
-      else if (!a.pl.n) a.tw = p->tw_adj[p->pass_of[0]];
+      else if (!a.pl) a.tw = p->tw_adj[p->pass_of[0]];
       a.cache = (fw->cache & PFK_KEEP_SRC ? PFK_KEEP_DST : 0) |
                 (fw->cache & PFK_KEEP_DST ? PFK_KEEP_SRC : 0);
       /* map roles: forward IN <-> adjoint OUT */
@@ -1122,10 +1133,8 @@ static int64_t batch_planes(const pa_plan *const *plans, int count) {
  * without a short-length pass, 5000 0.79 and 0.84. */
 static int batch_fuses(const pa_plan *p, int64_t planes) {
   if (!p->nfused || planes < PA_BATCH_PLANES) return 0;
-  const pfk_pass *col = &p->pass[p->pass_of[1]], *row = &p->pass[p->pass_of[2]];
   const int64_t points = p->n[1] * p->n[2];
-  return points >= 320 || planes <= 96 * points || !pfk_batch_short(col) ||
-         !pfk_batch_short(row);
+  return points >= 320 || planes <= 96 * points || !p->batch_short;
 }
 
 static pfk_batch *batch_build(const pa_plan *const *plans, int count) {

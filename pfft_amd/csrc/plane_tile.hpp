@@ -33,6 +33,7 @@ struct PlaneGeo {
   int n1, n2, pitch, nst, nrow, ntw1, ntw2;   // nrow: row stages; tables of rows, columns
   int keep_ld, keep_st;
   int64_t s1, d1;     // row strides
+  const void *twc;    // stage table of the columns
   PlaneStage st[PFK_PLANE_MAXST];
 };
 

@@ -4,6 +4,7 @@ short-length passes (the same lines and bytes, signs besides); parity of batches
 on both sides of the rule and of tiny planes in plans that run by themselves."""
 import time
 
+import numpy as np
 import pytest
 
 import pfft_amd as P
@@ -56,3 +57,26 @@ def test_tiny_planes_alone(n, prec):
     spec = spec_of("c2c", n)
     x = random_input(spec, 3)
     assert rel_l2(run_gpu(spec, x, prec=prec), oracle_out(spec, x)) < (1e-12 if prec == "f64" else 2e-6)
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_noalloc_planes_and_tiny_planes(prec):
+    # planes of several wave counts and three-pass plans in one fixed work-list,
+    # the geometries behind its tasks; a second call with other plans follows
+    rdt = np.float64 if prec == "f64" else np.float32
+    for sides in ([(64, 64), (4, 4), (20, 30), (16, 16), (7, 9), (96, 80)], [(8, 8), (30, 18)]):
+        work = []
+        for i in range(24):
+            spec = spec_of("c2c", [120, *sides[i % len(sides)]], sign=(-1) ** i)
+            x = random_input(spec, i)
+            a, b = (P.DeviceBuffer(x.size * np.dtype(rdt).itemsize) for _ in range(2))
+            a.upload(x.astype(rdt))
+            pl = P.Plan("c2c", spec.n, a.ptr, b.ptr, sign=spec.sign, comm=comm_for(2), prec=prec)
+            assert pl.ok
+            work.append((spec, x, a, b, pl))
+        assert P.execute_batch_noalloc([w[4] for w in work]) == 0
+        for spec, x, a, b, pl in work[:len(sides)] + work[-len(sides):]:
+            y = b.download(rdt, x.size).astype(np.float64)
+            assert rel_l2(y, oracle_out(spec, x)) < (1e-12 if prec == "f64" else 2e-6), spec.n
+        for w in work:
+            w[4].destroy()
