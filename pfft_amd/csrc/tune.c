@@ -63,14 +63,18 @@ static int g_timed = 0;   /* candidate timings performed (statistics) */
 
 /* Geometry key of a pass: everything that decides which launch is
  * fastest, nothing that only changes the values (twiddle pointers,
- * modulation starts). */
+ * modulation starts).  c: the cache marks, whose kernels are instantiations
+ * of their own; r: r2r kind and path, a kernel each.  (Selections of files
+ * written before these were part of the key match no pass and are timed
+ * again.) */
 static void pass_key(const pfk_pass *p, char *key) {
   int o = snprintf(key, PA_KEY_LEN,
-                   "k%d.p%d.n%lld.f%lld.i%lld@%lld.o%lld@%lld.s%lld:%lld.t%lld:%lld:%lld.h%d.m%d.mo%d%d",
+                   "k%d.p%d.n%lld.f%lld.i%lld@%lld.o%lld@%lld.s%lld:%lld.t%lld:%lld:%lld.h%d.m%d.mo%d%d.c%d.r%d:%d",
                    p->kind, p->prec, (long long)p->n, (long long)p->nf, (long long)p->nin,
                    (long long)p->zin, (long long)p->nout, (long long)p->zout, (long long)p->sin,
                    (long long)p->sout, (long long)p->text, (long long)p->tsin,
-                   (long long)p->tsout, p->hw, p->mfma, p->imod.on, p->omod.on);
+                   (long long)p->tsout, p->hw, p->mfma, p->imod.on, p->omod.on,
+                   p->cache, p->r2r, p->r2r_path);
   for (int b = 0; b < p->nb && o < PA_KEY_LEN; b++)
     o += snprintf(key + o, (size_t)(PA_KEY_LEN - o), ".b%lld:%lld:%lld", (long long)p->bext[b],
                   (long long)p->bsin[b], (long long)p->bsout[b]);
