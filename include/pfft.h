@@ -440,10 +440,13 @@ int pfft_amd_execute_batch_noalloc(const void *const *plans, int count);
  * fill arrays from the host. 0 on success. */
 int pfft_amd_memcpy_to_device(void *dst_dev, const void *src_host, size_t bytes);
 int pfft_amd_memcpy_to_host(void *dst_host, const void *src_dev, size_t bytes);
-/* Measurement hooks: number of device passes of a plan; mean duration
- * (ms) of each pass over `iters` runs on device arrays in/out (after one
- * untimed run) together with the bytes each pass reads plus writes; a text
- * description of the passes. */
+/* Measurement hooks: number of device passes of a plan, one per dimension;
+ * mean duration (ms) of each pass over `iters` runs on device arrays in/out
+ * (after one untimed run) together with the bytes each pass reads plus
+ * writes; a text description of the passes.  Where the plan by itself does
+ * two dimensions in one launch, that launch is what is timed: half of its
+ * time and bytes is given to each of the two passes, as in the plan's timer,
+ * and their lines of the description name it ("launch=1:plane"). */
 int pfft_amd_plan_npasses(const void *plan);
 int pfft_amd_time_passes(const void *plan, void *in, void *out, int iters, double *ms,
                          double *bytes);

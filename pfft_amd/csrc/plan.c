@@ -940,6 +940,18 @@ void pa_plan_destroy(pa_plan *p) {
 void *pa_plan_in(const pa_plan *p) { return p->in; }
 void *pa_plan_out(const pa_plan *p) { return p->out; }
 
+/* Adds a launch's time (or bytes) to the pass of its dimension, a plane's half
+ * and half to the passes of its two: inside a plane the stages of both
+ * dimensions alternate with no time of their own. */
+static void add_launch(const pa_plan *p, int fused, int launch, double v, double *per_pass) {
+  if (!fused) {
+    per_pass[launch] += v;
+  } else {
+    per_pass[p->pass_of[p->fdim[launch][0]]] += 0.5 * v;
+    per_pass[p->pass_of[p->fdim[launch][1]]] += 0.5 * v;
+  }
+}
+
 /* Runs the passes; `adjoint` runs them in reverse with swapped roles. */
 static void run(const pa_plan *p, void *in, void *out, int adjoint) {
   if (!p) return;
@@ -1020,19 +1032,16 @@ static void run(const pa_plan *p, void *in, void *out, int adjoint) {
   }
   if (!err && pfk_sync()) { pa_error("execution failed: %s", pfk_last_error()); err = 1; }
   if (!err && stamps) {
+    double per_pass[PA_MAXRNK] = {0};
     uint64_t end = 0;
     for (int i = PFK_STAMPS - PFK_STAMP_ENDS; i < PFK_STAMPS; i++)
       if (stamps[i] > end) end = stamps[i];
     for (int i = 0; i < np; i++) {
       const int k = adjoint ? np - 1 - i : i;
-      const double t = pfk_stamp_seconds(stamps[i], i + 1 < np ? stamps[i + 1] : end);
-      if (!fused) {
-        p->timer->trafo[p->tslot[k]] += t;
-      } else {   /* a plane's time: half to each of its dimensions */
-        p->timer->trafo[p->tslot[p->pass_of[p->fdim[k][0]]]] += 0.5 * t;
-        p->timer->trafo[p->tslot[p->pass_of[p->fdim[k][1]]]] += 0.5 * t;
-      }
+      add_launch(p, fused, k, pfk_stamp_seconds(stamps[i], i + 1 < np ? stamps[i + 1] : end),
+                 per_pass);
     }
+    for (int k = 0; k < p->npass; k++) p->timer->trafo[p->tslot[k]] += per_pass[k];
   } else if (!err && p->tev[0]) {
     for (int i = 0; i < p->npass; i++) {
       float ms = 0;
@@ -1294,44 +1303,42 @@ int pa_plans_execute_batch_noalloc(const pa_plan *const *plans, int count) {
   return 0;
 }
 
-/* Times every pass of the plan over `iters` back-to-back executions on
- * device arrays, after one untimed execution: one chain of HIP events on
- * the library stream, one between every two passes, read after a single
- * synchronisation.  (Reading the events after each execution would let the
- * stream run dry, and the next execution's first event would then carry
- * the host's launch latency into pass 0.)  ms[k] receives the mean
- * duration of pass k; bytes[k] the bytes pass k reads plus writes (one
- * sweep of its source and destination). */
+/* Times the launches of an execution (the fused ones where the plan by itself
+ * runs them) over `iters` back-to-back executions on device arrays, after one
+ * untimed execution: one chain of HIP events on the library stream, one between
+ * every two launches, read after a single synchronisation.  (Reading the events
+ * after each execution would let the stream run dry, and the next execution's
+ * first event would then carry the host's launch latency into pass 0.)  ms[k]
+ * receives the mean duration of pass k (add_launch); bytes[k] the bytes it
+ * reads plus writes (one sweep of its launch's source and destination). */
 int pa_plan_time_passes(const pa_plan *p, void *in, void *out, int iters, double *ms,
                         double *bytes) {
   if (!p || iters < 1 || !pfk_is_device_ptr(in) || !pfk_is_device_ptr(out)) return 1;
   void *bufs[4] = {in, out, p->scratch[0], p->scratch[1]};
-  const int nev = iters * p->npass + 1;
+  const int fused = p->fused_alone, np = prog_n(p, fused);
+  const int nev = iters * np + 1;
   void **ev = (void **)calloc((size_t)nev, sizeof(void *));
   if (!ev) return 1;
   int err = 0, made = 0;
   for (; made < nev && !err; made++)
     if (pfk_event_create(&ev[made])) err = 1;
-  for (int k = 0; k < p->npass && !err; k++)
-    err = pfk_launch_pass(&p->pass[k], bufs[p->src_role[k]], bufs[p->dst_role[k]]);
-  if (!err) err = pfk_event_record(ev[0]);
-  for (int it = 0; it < iters && !err; it++)
-    for (int k = 0; k < p->npass && !err; k++) {
-      err = pfk_launch_pass(&p->pass[k], bufs[p->src_role[k]], bufs[p->dst_role[k]]);
-      if (!err) err = pfk_event_record(ev[it * p->npass + k + 1]);
+  for (int it = -1; it < iters && !err; it++)
+    for (int i = 0; i < np && !err; i++) {
+      if (it == 0 && i == 0) err = pfk_event_record(ev[0]);
+      if (!err)
+        err = pfk_launch_pass(prog_pass(p, fused, i), bufs[prog_src(p, fused, i)],
+                              bufs[prog_dst(p, fused, i)]);
+      if (!err && it >= 0) err = pfk_event_record(ev[it * np + i + 1]);
     }
-  for (int k = 0; k < p->npass; k++) ms[k] = 0;
+  for (int k = 0; k < p->npass; k++) ms[k] = bytes[k] = 0;
   for (int it = 0; it < iters && !err; it++)
-    for (int k = 0; k < p->npass && !err; k++) {
+    for (int i = 0; i < np && !err; i++) {
       float t = 0;
-      const int e0 = it * p->npass + k;
+      const int e0 = it * np + i;
       if (pfk_event_elapsed_ms(ev[e0], ev[e0 + 1], &t)) err = 1;
-      ms[k] += t;
+      add_launch(p, fused, i, t / iters, ms);
     }
-  for (int k = 0; k < p->npass; k++) {
-    ms[k] /= iters;
-    bytes[k] = pa_pass_bytes(&p->pass[k]);
-  }
+  for (int i = 0; i < np; i++) add_launch(p, fused, i, pa_pass_bytes(prog_pass(p, fused, i)), bytes);
   for (int i = 0; i < made; i++)
     if (ev[i]) pfk_event_destroy(ev[i]);
   free(ev);
@@ -1342,6 +1349,7 @@ int pa_plan_npasses(const pa_plan *p) { return p ? p->npass : 0; }
 
 static const char *kernel_name(const pfk_pass *ps) {
   if (ps->kind == PFK_COPY) return "copy";
+  if (ps->pl) return "plane";
   if (ps->n1) return "long-two-step";
   if (ps->r2r_path)
     return (pfk_pass_kernels(ps) & PFK_HAS_MIXED) ? "r2r-mixed" : "r2r-inner-fft";
@@ -1365,27 +1373,35 @@ static const char *kernel_name(const pfk_pass *ps) {
   return (fam & PFK_HAS_MIXED) ? "mixed" : "general";
 }
 
+static const char *xcd_name(const pfk_pass *ps) {
+  const char *name = kernel_name(ps);
+  return ps->xcd_remap && (!strncmp(name, "fast", 4) || !strcmp(name, "mixed")) ? "+xcd" : "";
+}
+
 /* One line per pass: kind, length, strides, batch and tile geometry,
- * the kernel that runs it. */
+ * the kernel that runs it.  Where the plan by itself runs fused launches
+ * instead, "launch=i:name" is the one that does the pass's dimension (the
+ * rest of the line is the pass as batches may run it). */
 int pa_plan_describe(const pa_plan *p, char *buf, size_t len) {
   static const char *kn[] = {"c2c", "r2c", "c2r", "copy", "r2r"};   /* enum pfk_kind */
   size_t o = 0;
   buf[0] = 0;
   for (int k = 0; k < p->npass && o < len; k++) {
     const pfk_pass *ps = &p->pass[k];
+    char launch[64] = "";
+    for (int i = 0; p->fused_alone && i < p->nfused; i++)
+      if (p->pass_of[p->fdim[i][0]] == k || p->pass_of[p->fdim[i][1]] == k)
+        snprintf(launch, sizeof launch, " launch=%d:%s%s", i, kernel_name(&p->fused[i]),
+                 xcd_name(&p->fused[i]));
     o += (size_t)snprintf(buf + o, len - o,
                           "pass %d: %s n=%lld nf=%lld nin=%lld@%lld nout=%lld@%lld sin=%lld "
-                          "sout=%lld tile=%lld(%lld,%lld) nb=%d roles=%d->%d kernel=%s%s\n",
+                          "sout=%lld tile=%lld(%lld,%lld) nb=%d roles=%d->%d%s kernel=%s%s\n",
                           k, (ps->kind >= 0 && ps->kind <= PFK_R2R) ? kn[ps->kind] : "?",
                           (long long)ps->n, (long long)ps->nf,
                           (long long)ps->nin, (long long)ps->zin, (long long)ps->nout,
                           (long long)ps->zout, (long long)ps->sin, (long long)ps->sout,
                           (long long)ps->text, (long long)ps->tsin, (long long)ps->tsout, ps->nb,
-                          p->src_role[k], p->dst_role[k], kernel_name(ps),
-                          (ps->xcd_remap && (!strncmp(kernel_name(ps), "fast", 4) ||
-                                             !strcmp(kernel_name(ps), "mixed")))
-                              ? "+xcd"
-                              : "");
+                          p->src_role[k], p->dst_role[k], launch, kernel_name(ps), xcd_name(ps));
   }
   return 0;
 }

@@ -172,6 +172,7 @@ double pa_pass_bytes(const pfk_pass *ps) {
   const double dst_sz = (ps->kind == PFK_C2R || ps->kind == PFK_R2R) ? rs : 2 * rs;
   double nl = (double)ps->text;
   for (int b = 0; b < ps->nb; b++) nl *= (double)ps->bext[b];
+  if (ps->pl) nl *= (double)ps->pl->n;
   return nl * ((double)ps->nin * src_sz + (double)ps->nout * dst_sz);
 }
 
