@@ -86,6 +86,13 @@ void pa_plan_info(const pa_plan *p, int *rnk_n, const INT **n, const INT **ni, c
 /* ---- autotuner and wisdom (tune.c) ---- */
 int pa_tune_lookup(pfk_pass *ps, unsigned effort);
 int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort);
+typedef struct pa_launch {
+  const pfk_pass *ps;
+  const void *src;
+  void *dst;
+} pa_launch;
+int pa_tune_planes(pfk_pass *plane, const pa_launch *fused, int nfused, const pa_launch *passes,
+                   int npasses, unsigned effort);
 double pa_pass_bytes(const pfk_pass *ps);
 int pa_wisdom_export(const char *filename);
 int pa_wisdom_import(const char *filename);

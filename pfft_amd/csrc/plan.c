@@ -338,7 +338,19 @@ static void tune_plan(pa_plan *p) {
   const unsigned effort = p->pfft_flags & (PFFT_ESTIMATE | PFFT_PATIENT | PFFT_EXHAUSTIVE);
   int open_[PA_MAXRNK] = {0}, any = 0;
   for (int k = 0; k < p->npass; k++) any |= open_[k] = pa_tune_lookup(&p->pass[k], effort);
-  if (!any) return;
+  /* a plan that would run planes: the plane against one pass per dimension, and the
+   * pass beside it */
+  pfk_pass *plane = NULL, *line = NULL;
+  int open_plane = 0, open_line = 0;
+  if (p->fused_alone) {
+    const int i = p->fused[0].pl ? 0 : 1;
+    plane = &p->fused[i];
+    line = &p->fused[1 - i];
+    open_plane = pa_tune_lookup(plane, effort);
+    p->fused_alone = open_plane || plane->variant == 9;
+    if (p->fused_alone) open_line = pa_tune_lookup(line, effort);
+  }
+  if (!any && !open_plane && !open_line) return;
   void *tin = NULL, *tout = NULL;
   const size_t ib = (size_t)(p->in_elems * (int64_t)p->in_esz);
   const size_t ob = (size_t)(p->out_elems * (int64_t)p->out_esz);
@@ -353,6 +365,19 @@ static void tune_plan(pa_plan *p) {
     if (open_[k] &&
         pa_tune_measure(&p->pass[k], bufs[p->src_role[k]], bufs[p->dst_role[k]], effort))
       break;
+  if (open_line) {
+    const int i = line == &p->fused[1];
+    (void)pa_tune_measure(line, bufs[p->fsrc[i]], bufs[p->fdst[i]], effort);
+  }
+  if (open_plane) {
+    pa_launch two[2], each[PA_MAXRNK];
+    for (int i = 0; i < 2; i++)
+      two[i] = (pa_launch){&p->fused[i], bufs[p->fsrc[i]], bufs[p->fdst[i]]};
+    for (int k = 0; k < p->npass; k++)
+      each[k] = (pa_launch){&p->pass[k], bufs[p->src_role[k]], bufs[p->dst_role[k]]};
+    (void)pa_tune_planes(plane, two, 2, each, p->npass, effort);
+    p->fused_alone = plane->variant == 9;
+  }
   (void)pfk_sync();
   pfk_free(tin);
   pfk_free(tout);
@@ -446,7 +471,7 @@ static void fuse_planes(pa_plan *p, const arrgeo *geo, const int *ord) {
       if (fill_geometry(q, S, D, 0) || check_bounds(q)) return;
       p->fdim[i][0] = p->fdim[i][1] = 0;
     }
-    q->variant = 0;
+    q->variant = q->pl ? 9 : 0;   /* 9: planes (tune.c) */
     q->cache = cache_policy(q, i == 0, i == 1);
   }
   p->nfused = 2;
@@ -454,7 +479,7 @@ static void fuse_planes(pa_plan *p, const arrgeo *geo, const int *ord) {
    * are CUs, and two planes a CU.  Pairs against three passes: complex128
    * 64x64x64 61 / 53 us, 256x64x64 75 / 80, 300x50x60 84 / 96, 256x16x200 70 /
    * 85; complex64 1000x100x100 (one plane a CU) 293 / 234, 512x128x128 180 /
-   * 178, 300x50x60 72 / 87. */
+   * 178, 300x50x60 72 / 87.  Tuned plans time both (tune_plan). */
   p->fused_alone = p->n[0] >= 192 && pfk_plane_covers(&p->fused[plane_first ? 0 : 1]) <= 72 * 1024;
 }
 

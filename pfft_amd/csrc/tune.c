@@ -23,6 +23,8 @@
  *   (9,0) (9,1) the mixed-radix kernel, where the power-of-two kernels do not
  *         reach or the tile dimension fills less than one of their tiles;
  *   (1,0) the general kernel, where the mixed-radix one is no candidate.
+ * A plane pass (pfk_plane) is (9,0) where its plan runs it and (0,0) where three
+ * passes were faster.
  * A pass with one candidate is not timed.  All candidates compute the
  * same transform (the power-of-two variants bit-identically, the others
  * with their own factorisations).  A pass run by an MFMA kernel keeps it
@@ -75,6 +77,9 @@ static void pass_key(const pfk_pass *p, char *key) {
                    (long long)p->sout, (long long)p->text, (long long)p->tsin,
                    (long long)p->tsout, p->hw, p->mfma, p->imod.on, p->omod.on,
                    p->cache, p->r2r, p->r2r_path);
+  if (p->pl)
+    o += snprintf(key + o, (size_t)(PA_KEY_LEN - o), ".q%lld:%lld:%lld", (long long)p->pl->n,
+                  (long long)p->pl->sin, (long long)p->pl->sout);
   for (int b = 0; b < p->nb && o < PA_KEY_LEN; b++)
     o += snprintf(key + o, (size_t)(PA_KEY_LEN - o), ".b%lld:%lld:%lld", (long long)p->bext[b],
                   (long long)p->bsin[b], (long long)p->bsout[b]);
@@ -176,19 +181,28 @@ double pa_pass_bytes(const pfk_pass *ps) {
   return nl * ((double)ps->nin * src_sz + (double)ps->nout * dst_sz);
 }
 
-/* Mean duration of `reps` launches after one warm-up launch; < 0 on a
- * launch error. */
-static double time_launches(const pfk_pass *ps, const void *src, void *dst, int reps, void *e0,
-                            void *e1) {
-  if (pfk_launch_pass(ps, src, dst)) return -1;
+static int launch_chain(const pa_launch *l, int n) {
+  for (int k = 0; k < n; k++)
+    if (pfk_launch_pass(l[k].ps, l[k].src, l[k].dst)) return 1;
+  return 0;
+}
+
+/* Mean duration of `reps` runs of the launches l[0..n-1] after one warm-up
+ * run; < 0 on a launch error. */
+static double time_launches(const pa_launch *l, int n, int reps, void *e0, void *e1) {
+  if (launch_chain(l, n)) return -1;
   if (pfk_event_record(e0)) return -1;
   for (int i = 0; i < reps; i++)
-    if (pfk_launch_pass(ps, src, dst)) return -1;
+    if (launch_chain(l, n)) return -1;
   if (pfk_event_record(e1)) return -1;
   float t = 0;
   if (pfk_event_elapsed_ms(e0, e1, &t)) return -1;
   g_timed++;
   return (double)t / reps;
+}
+
+static int effort_reps(unsigned effort) {
+  return (effort & PFFT_EXHAUSTIVE) ? 10 : (effort & PFFT_PATIENT) ? 6 : 3;
 }
 
 /* Settles a pass without timing where possible: returns 0 if the pass
@@ -201,7 +215,7 @@ int pa_tune_lookup(pfk_pass *ps, unsigned effort) {
   const int mode = ev ? atoi(ev) : 1;   /* 0 off, 1 on, 2 on for every pass size */
   if (mode == 0 || (effort & PFFT_ESTIMATE) || ps->kind == PFK_COPY) return 0;
   const int fam = pfk_pass_kernels(ps);
-  if (fam == 0) return 0;   /* general kernel only */
+  if (fam == 0 && !ps->pl) return 0;   /* general kernel only */
   if (mode != 2 && pa_pass_bytes(ps) < PA_TUNE_MIN_BYTES) return 0;
   wisdom_env_load();
   char key[PA_KEY_LEN];
@@ -222,7 +236,7 @@ int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort) {
   pass_key(ps, key);
   const char *rv = getenv("PFFT_AMD_XCD_REMAP");
   const int remap_fixed = (rv && *rv) ? (rv[0] == '1') : -1;
-  const int reps = (effort & PFFT_EXHAUSTIVE) ? 10 : (effort & PFFT_PATIENT) ? 6 : 3;
+  const int reps = effort_reps(effort);
   static const int cand[16][2] = {{0, 0}, {0, 1}, {2, 0},  {2, 1},  {4, 0},  {4, 1},  {6, 0},
                                   {6, 1}, {8, 0}, {8, 1}, {12, 0}, {12, 1}, {3, 0}, {9, 0},
                                   {9, 1}, {1, 0}};
@@ -257,7 +271,8 @@ int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort) {
     if ((pow2 || v == 9) && remap_fixed >= 0 && r != remap_fixed) continue;
     ps->variant = v;
     ps->xcd_remap = r;
-    const double t = time_launches(ps, src, dst, reps, e0, e1);
+    const pa_launch l = {ps, src, dst};
+    const double t = time_launches(&l, 1, reps, e0, e1);
     if (t < 0) { err = 1; break; }
     if (best < 0 || t < best) { best = t; best_v = v; best_r = r; }
   }
@@ -272,5 +287,29 @@ int pa_tune_measure(pfk_pass *ps, const void *src, void *dst, unsigned effort) {
   ps->variant = best_v;
   ps->xcd_remap = best_r;
   if (!wisdom_put(key, best_v, best_r, best)) wisdom_env_save();
+  return 0;
+}
+
+/* Times the launches of an execution with the plane pass against those of
+ * one pass per dimension and keeps the faster in the plane's variant (9: planes,
+ * 0: one pass per dimension) and in the wisdom cache.  On a device error the
+ * plane keeps its default. */
+int pa_tune_planes(pfk_pass *plane, const pa_launch *fused, int nfused, const pa_launch *passes,
+                   int npasses, unsigned effort) {
+  char key[PA_KEY_LEN];
+  pass_key(plane, key);
+  const int reps = effort_reps(effort);
+  void *e0 = NULL, *e1 = NULL;
+  if (pfk_event_create(&e0) || pfk_event_create(&e1)) {
+    if (e0) pfk_event_destroy(e0);
+    return 1;
+  }
+  const double tp = time_launches(fused, nfused, reps, e0, e1);
+  const double td = tp < 0 ? -1 : time_launches(passes, npasses, reps, e0, e1);
+  pfk_event_destroy(e0);
+  pfk_event_destroy(e1);
+  if (pfk_sync() || td < 0) return 1;
+  plane->variant = tp <= td ? 9 : 0;
+  if (!wisdom_put(key, plane->variant, 0, tp <= td ? tp : td)) wisdom_env_save();
   return 0;
 }
