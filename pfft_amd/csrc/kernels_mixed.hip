@@ -88,6 +88,11 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
   // Halved while the tile exceeds 80 KiB (two workgroups per CU) or 512 threads,
   // and, down to the segment (two lines along the lines), while the pass has
   // fewer than two tiles per CU.  A matrix-core stage takes 8 lines at least.
+  // r2r tiles go below the segment, to 4 lines, while the pass has fewer than two
+  // tiles per CU: such a pass is bound by what one workgroup does to one tile
+  // (single-precision plans, three launches a pass / segments / 4 lines: 1024x128x2
+  // 83 / 79 / 61 us with kinds up to 1.23 times the three launches, 128x128x8 94 /
+  // 81 / 56, 64x64x64 85 / 62 / 45; 8 lines 70, 65, 45).
   int64_t lines = p->text;
   for (int i = 0; i < p->nb; i++) lines *= p->bext[i];
   const int cmin = g->big ? 8 : 1;
@@ -98,6 +103,7 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
   while (C < 64 && (size_t)(2 * C) * rows * esz <= tile) C *= 2;
   if (C < cmin) C = cmin;
   while (C > cseg && lines < 512 * (int64_t)C) C /= 2;
+  bool few = false;
   for (;; C /= 2) {
     // row pitch of 2 slots modulo the 256 bytes of a bank cycle, so that 8 (16)
     // lines x 2 positions spread over all banks; consecutive positions do anyway,
@@ -130,9 +136,12 @@ static int mixed_geo(const pfk_pass *p, MixGeo *g, const void *src, const void *
     // r2r lines too long for half a segment, or with matrix-core stages, keep the
     // three launches
     if (r2r && g->big) return 0;
-    if (r2r && !(g->lm_ld && g->lm_st) && C < seg / 2) return 0;
-    if ((nt <= 512 && lds <= 80 * 1024) || (C == cmin && nt <= 512 && lds <= 158 * 1024))
-      return nt;
+    if (r2r && !(g->lm_ld && g->lm_st) && C < seg / 2 && !few) return 0;
+    if ((nt <= 512 && lds <= 80 * 1024) || (C == cmin && nt <= 512 && lds <= 158 * 1024)) {
+      if (!r2r || C <= 4 || lines >= 512 * (int64_t)C) return nt;
+      few = true;
+      continue;
+    }
     if (C == cmin) return 0;
   }
 }
