@@ -55,7 +55,7 @@ static int64_t slots_per_line(const pfk_pass *p) {
 int generic_tiling(const pfk_pass *p, int *Cout, int *pitch_out, size_t *lds_out) {
   constexpr int NT = 256, EPT = 16;
   const int64_t ns = slots_per_line(p);
-  const int64_t nf = (p->kind == PFK_COPY) ? 1 : p->nf;
+  const int64_t nf = (p->kind == PFK_COPY || p->kind == PFK_COPY_REAL) ? 1 : p->nf;
   const size_t esz = (p->prec == PFK_F64) ? 16 : 8;
   int C = 64;
   while (C > 1 && (C * nf > (int64_t)NT * EPT || C * (ns + 1) * (int64_t)esz > g_max_lds ||
@@ -103,6 +103,10 @@ static int launch_generic_t(const pfk_pass *p, const void *src, void *dst) {
       case PFK_R2R:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_R2R, EPT>), grid, block, lds, g_stream, *p, C,
                            (int)pitch, base, ntiles, s, d);
+        break;
+      case PFK_COPY_REAL:
+        hipLaunchKernelGGL((k_pass_generic<T, PFK_COPY_REAL, EPT>), grid, block, lds, g_stream, *p,
+                           C, (int)pitch, base, ntiles, s, d);
         break;
       default:
         hipLaunchKernelGGL((k_pass_generic<T, PFK_COPY, EPT>), grid, block, lds, g_stream, *p, C,

@@ -110,6 +110,24 @@ __device__ __forceinline__ void pass_tile(const pfk_pass &P, const int C, const 
           const T f = (T)mod_sign(P.imod, j);
           buf[cc * pitch + zin + j] = C2{v.x * f, v.y * f};
         });
+  } else if (KIND == PFK_COPY_REAL) {
+    if (nin < n)
+      for (int idx = tid; idx < nl * n; idx += NT) {
+        const int cc = idx / n, p = idx - cc * n;
+        if (p < zin || p >= zin + nin) buf[cc * pitch + p] = C2{0, 0};
+      }
+    batched<8, T>(
+        tid, NT, nl * nin,
+        [&](int idx) {
+          const int cc = ld_tile_fast ? idx % nl : idx / nin;
+          const int j = ld_tile_fast ? idx / nl : idx % nin;
+          return src[sb + cc * P.tsin + (int64_t)j * P.sin];
+        },
+        [&](int idx, T v) {
+          const int cc = ld_tile_fast ? idx % nl : idx / nin;
+          const int j = ld_tile_fast ? idx / nl : idx % nin;
+          buf[cc * pitch + zin + j] = C2{v * (T)mod_sign(P.imod, j), 0};
+        });
   } else if (KIND == PFK_R2R) {
     // real line x (length n, embedded at zin) -> extended real sequence u of
     // length nf in complex slots (layout in pfk.h)
@@ -271,7 +289,7 @@ __device__ __forceinline__ void pass_tile(const pfk_pass &P, const int C, const 
   }
 
   // ---------------- FFT stages (output-centric Stockham) ----------------
-  if (KIND != PFK_COPY) {
+  if (KIND != PFK_COPY && KIND != PFK_COPY_REAL) {
     int L = 1;
     for (int s = 0; s < P.nstages; ++s) {
       const int R = P.radix[s];
@@ -353,6 +371,14 @@ __device__ __forceinline__ void pass_tile(const pfk_pass &P, const int C, const 
       const C2 v = buf[cc * pitch + zout + k];
       const T f = (T)mod_sign(P.omod, k);
       d[db + cc * P.tsout + (int64_t)k * P.sout] = C2{v.x * f, v.y * f};
+    }
+  } else if (KIND == PFK_COPY_REAL) {
+    for (int idx = tid; idx < nl * nout; idx += NT) {
+      int cc, k;
+      if (st_tile_fast) { cc = idx % nl; k = idx / nl; }
+      else { k = idx % nout; cc = idx / nout; }
+      dst[db + cc * P.tsout + (int64_t)k * P.sout] =
+          buf[cc * pitch + zout + k].x * (T)mod_sign(P.omod, k);
     }
   } else if (KIND == PFK_R2R) {
     const int kd = P.r2r;

@@ -45,7 +45,8 @@ extern "C" {
 #define PFK_MAXSTAGES 24
 #define PFK_MIX_MAXST 7   /* stages of the mixed-radix kernel */
 
-enum pfk_kind { PFK_C2C = 0, PFK_R2C = 1, PFK_C2R = 2, PFK_COPY = 3, PFK_R2R = 4 };
+/* PFK_COPY, PFK_COPY_REAL: a skipped dimension of complex, of real arrays */
+enum pfk_kind { PFK_C2C = 0, PFK_R2C = 1, PFK_C2R = 2, PFK_COPY = 3, PFK_R2R = 4, PFK_COPY_REAL = 5 };
 
 /* Real-to-real kinds of a PFK_R2R pass (the FFTW kind numbers of
  * include/pfft.h).  A length-n r2r line is computed as a forward complex

@@ -412,7 +412,7 @@ static INT r2r_length(int kind, INT n) {
 static int cache_policy(const pfk_pass *ps, int first, int last) {
   const double keep_user = 80.0 * 1048576, keep_mid = 288.0 * 1048576;
   const double rsz = ps->prec == PFK_F64 ? 8 : 4;
-  const int r2r = ps->kind == PFK_R2R;
+  const int r2r = ps->kind == PFK_R2R || ps->kind == PFK_COPY_REAL;
   const double sb = (double)ps->src_elems * rsz * (ps->kind == PFK_R2C || r2r ? 1 : 2);
   const double db = (double)ps->dst_elems * rsz * (ps->kind == PFK_C2R || r2r ? 1 : 2);
   if (sb < 16.0 * 1048576 && db < 16.0 * 1048576) return 0;
@@ -722,7 +722,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
     int kind = PFK_C2C;
     if (d == last && is_r2c) kind = PFK_R2C;
     else if (d == last && is_c2r) kind = PFK_C2R;
-    else if (skipped) kind = PFK_COPY;
+    else if (skipped) kind = is_r2r ? PFK_COPY_REAL : PFK_COPY;
     else if (is_r2r) kind = PFK_R2R;
     ps->kind = kind;
     ps->xcd_remap = xcd_remap;
@@ -773,7 +773,8 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
           !pfk_pass_check(&in))
         ps->r2r_path = path;
     }
-    if (kind != PFK_COPY && !ps->r2r_path && ps->nf > PFK_MAXLINE) {
+    const int copy = kind == PFK_COPY || kind == PFK_COPY_REAL;
+    if (!copy && !ps->r2r_path && ps->nf > PFK_MAXLINE) {
       /* long lines: two steps through a work buffer (c2c; even-length
        * r2c / c2r as their half-length complex line) */
       if ((kind == PFK_R2C || kind == PFK_C2R) && n[d] % 2) {
@@ -788,7 +789,7 @@ pa_plan *pa_plan_create(int prec, int rnk_n, const INT *n, const INT *ni, const 
         goto fail;
       }
     }
-    if (kind != PFK_COPY) {
+    if (!copy) {
       ps->nstages = pfk_factorize(ps->nf, ps->radix);
       if (ps->nstages < 0) { pa_error("cannot factor length %lld", (long long)ps->nf); goto fail; }
       if (ps->r2r_path) {
@@ -1373,7 +1374,7 @@ int pa_plan_time_passes(const pa_plan *p, void *in, void *out, int iters, double
 int pa_plan_npasses(const pa_plan *p) { return p ? p->npass : 0; }
 
 static const char *kernel_name(const pfk_pass *ps) {
-  if (ps->kind == PFK_COPY) return "copy";
+  if (ps->kind == PFK_COPY || ps->kind == PFK_COPY_REAL) return "copy";
   if (ps->pl) return "plane";
   if (ps->n1) return "long-two-step";
   if (ps->r2r_path)
@@ -1408,7 +1409,7 @@ static const char *xcd_name(const pfk_pass *ps) {
  * instead, "launch=i:name" is the one that does the pass's dimension (the
  * rest of the line is the pass as batches may run it). */
 int pa_plan_describe(const pa_plan *p, char *buf, size_t len) {
-  static const char *kn[] = {"c2c", "r2c", "c2r", "copy", "r2r"};   /* enum pfk_kind */
+  static const char *kn[] = {"c2c", "r2c", "c2r", "copy", "r2r", "copy"};   /* enum pfk_kind */
   size_t o = 0;
   buf[0] = 0;
   for (int k = 0; k < p->npass && o < len; k++) {
@@ -1421,7 +1422,7 @@ int pa_plan_describe(const pa_plan *p, char *buf, size_t len) {
     o += (size_t)snprintf(buf + o, len - o,
                           "pass %d: %s n=%lld nf=%lld nin=%lld@%lld nout=%lld@%lld sin=%lld "
                           "sout=%lld tile=%lld(%lld,%lld) nb=%d roles=%d->%d%s kernel=%s%s\n",
-                          k, (ps->kind >= 0 && ps->kind <= PFK_R2R) ? kn[ps->kind] : "?",
+                          k, (ps->kind >= 0 && ps->kind <= PFK_COPY_REAL) ? kn[ps->kind] : "?",
                           (long long)ps->n, (long long)ps->nf,
                           (long long)ps->nin, (long long)ps->zin, (long long)ps->nout,
                           (long long)ps->zout, (long long)ps->sin, (long long)ps->sout,

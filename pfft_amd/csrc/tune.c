@@ -173,8 +173,9 @@ static void wisdom_env_save(void) {
 
 double pa_pass_bytes(const pfk_pass *ps) {
   const double rs = (ps->prec == PFK_F64) ? 8.0 : 4.0;
-  const double src_sz = (ps->kind == PFK_R2C || ps->kind == PFK_R2R) ? rs : 2 * rs;
-  const double dst_sz = (ps->kind == PFK_C2R || ps->kind == PFK_R2R) ? rs : 2 * rs;
+  const int real = ps->kind == PFK_R2R || ps->kind == PFK_COPY_REAL;
+  const double src_sz = (ps->kind == PFK_R2C || real) ? rs : 2 * rs;
+  const double dst_sz = (ps->kind == PFK_C2R || real) ? rs : 2 * rs;
   double nl = (double)ps->text;
   for (int b = 0; b < ps->nb; b++) nl *= (double)ps->bext[b];
   if (ps->pl) nl *= (double)ps->pl->n;
@@ -213,7 +214,9 @@ static int effort_reps(unsigned effort) {
 int pa_tune_lookup(pfk_pass *ps, unsigned effort) {
   const char *ev = getenv("PFFT_AMD_TUNE");
   const int mode = ev ? atoi(ev) : 1;   /* 0 off, 1 on, 2 on for every pass size */
-  if (mode == 0 || (effort & PFFT_ESTIMATE) || ps->kind == PFK_COPY) return 0;
+  if (mode == 0 || (effort & PFFT_ESTIMATE) || ps->kind == PFK_COPY ||
+      ps->kind == PFK_COPY_REAL)
+    return 0;
   const int fam = pfk_pass_kernels(ps);
   if (fam == 0 && !ps->pl) return 0;   /* general kernel only */
   if (mode != 2 && pa_pass_bytes(ps) < PA_TUNE_MIN_BYTES) return 0;
