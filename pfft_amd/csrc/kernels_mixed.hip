@@ -13,10 +13,6 @@ int launch_mixed_r2r_f64(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
 int launch_mixed_r2r_f32(const pfk_pass *p, const MixGeo &g, int nt, size_t lds,
                          const void *src, void *dst);
 
-static uint32_t recip(int64_t d) {   // div_m
-  return d <= 1 ? 0 : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
-}
-
 static size_t mix_lds(const MixGeo *g, size_t esz) {
   return (size_t)g->C * (32 + (size_t)(g->big + 1) * g->pitch * esz) + (size_t)g->ntw * esz;
 }

@@ -25,10 +25,6 @@ k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const T *__re
   stamp_end(P, nplanes - 1 - (id - gridDim.x));
 }
 
-static uint32_t recip(int64_t d) {
-  return d <= 1 ? 0 : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
-}
-
 static size_t plane_lds(const pfk_pass *p, PlaneGeo *g) {
   g->n1 = (int)p->pl->n;
   g->n2 = (int)p->nf;

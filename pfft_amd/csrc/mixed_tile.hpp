@@ -70,11 +70,6 @@ constexpr int mix_kind_r2r(int r2r) { return 16 + r2r; }
 constexpr bool mix_r2r(int kind) { return kind >= 16; }
 constexpr int mix_r2r_kind(int kind) { return kind - 16; }
 
-// i / d for i * d < 2^32 with m = ceil(2^32 / d) (m = 0: d = 1)
-__device__ __forceinline__ int div_m(int i, uint32_t m) {
-  return m ? (int)__umulhi((uint32_t)i, m) : i;
-}
-
 template <typename T>
 struct MixCtx {
   const pfk_pass &P;
@@ -424,7 +419,7 @@ __device__ __forceinline__ void mix_stage(const MixCtx<T> &X, const int s) {
 #pragma unroll
   for (int i = 0; i < I; ++i) dft_any<R, -1>(v[i]);
   if (last && !z_lds && KIND != PFK_R2C && (G.plain || G.vec)) {
-        const int64_t sout = KIND == PFK_C2C ? X.P.sout : 1, step = NB * sout;
+    const int64_t sout = KIND == PFK_C2C ? X.P.sout : 1, step = NB * sout;
 #pragma unroll
     for (int i = 0; i < I; ++i) {
       if (cs[i] >= X.nl) continue;

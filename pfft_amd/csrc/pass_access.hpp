@@ -68,6 +68,14 @@ __device__ __forceinline__ T msign(const pfk_mod &m, int64_t j) {
   return (T)s;
 }
 
+// i / d for i * d < 2^32, with m = recip(d) (m = 0: d = 1)
+__device__ __forceinline__ int div_m(int i, uint32_t m) {
+  return m ? (int)__umulhi((uint32_t)i, m) : i;
+}
+static inline uint32_t recip(int64_t d) {   // ceil(2^32 / d)
+  return d <= 1 ? 0 : (uint32_t)((((uint64_t)1 << 32) + (uint64_t)d - 1) / (uint64_t)d);
+}
+
 struct TileCtx {
   int64_t sb, db;
   int64_t c0;   // first line of the tile along the tile dimension

@@ -37,10 +37,6 @@ struct PlaneGeo {
   PlaneStage st[PFK_PLANE_MAXST];
 };
 
-__device__ __forceinline__ int plane_div(int i, uint32_t m) {   // i / d, m = ceil(2^32 / d)
-  return m ? (int)__umulhi((uint32_t)i, m) : i;
-}
-
 // one slot of padding per 16 positions of a row spreads the row stages' strided
 // stores over the banks
 __device__ __forceinline__ int plane_slot(const PlaneGeo &G, int row, int x) {
@@ -65,10 +61,10 @@ __device__ __forceinline__ void plane_stage(const PlaneGeo &G, const int s, cons
 #pragma unroll
     for (int i = 0; i < I; ++i) {
       const int it0 = tid + i * NT, it = it0 < items ? it0 : 0;
-      const int hi = plane_div(it, S.mdiv), lo = it - hi * (col ? W : NB);
+      const int hi = div_m(it, S.mdiv), lo = it - hi * (col ? W : NB);
       cs[i] = c0 + (col ? lo : hi);
       bs[i] = col ? hi : lo;
-      ks[i] = bs[i] - plane_div(bs[i], S.mlen) * L;
+      ks[i] = bs[i] - div_m(bs[i], S.mlen) * L;
       const bool ok = it0 < items && cs[i] < total;
       if (!ok) { cs[i] = c0; bs[i] = 0; ks[i] = -1; }   // reads line c0, writes nothing
     }
