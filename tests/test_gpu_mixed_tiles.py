@@ -10,6 +10,7 @@ import pfft_amd as P
 from gpu_util import spec_of, random_input, run_gpu, oracle_out, out_mask, rel_l2
 from test_gpu_tune import _plan_lines, _rewrite, tune_all   # noqa: F401 (fixture)
 from test_gpu_mixed import KINDS
+from shared_comm import shared_comm   # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 TI, TO = P.TRANSPOSED_IN, P.TRANSPOSED_OUT

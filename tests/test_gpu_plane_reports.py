@@ -10,6 +10,7 @@ import pytest
 import pfft_amd as P
 from gpu_util import spec_of, random_input, run_gpu, oracle_out, rel_l2
 from test_gpu_timer import timer_vec
+from shared_comm import shared_comm   # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 

@@ -7,9 +7,11 @@ import time
 import numpy as np
 import pytest
 
+import gpu_util
 import pfft_amd as P
-from gpu_util import spec_of, random_input, run_gpu, oracle_out, rel_l2, comm_for
+from gpu_util import spec_of, random_input, run_gpu, oracle_out, rel_l2
 from test_gpu_plane import run_batch
+from shared_comm import shared_comm   # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -17,8 +19,8 @@ pytestmark = pytest.mark.gpu
 def batch_us(n, count, prec, flags):
     pts = 2 * n[0] * n[1] * n[2] * (8 if prec == "f64" else 4)
     bufs = [(P.DeviceBuffer(pts), P.DeviceBuffer(pts)) for _ in range(count)]
-    plans = [P.Plan("c2c", n, a.ptr, b.ptr, flags=flags, comm=comm_for(2), prec=prec)
-             for a, b in bufs]
+    comm = gpu_util.comm_for(2)
+    plans = [P.Plan("c2c", n, a.ptr, b.ptr, flags=flags, comm=comm, prec=prec) for a, b in bufs]
     assert all(p.ok for p in plans)
     best = 1e9
     for _ in range(20):
@@ -64,6 +66,7 @@ def test_noalloc_planes_and_tiny_planes(prec):
     # planes of several wave counts and three-pass plans in one fixed work-list,
     # the geometries behind its tasks; a second call with other plans follows
     rdt = np.float64 if prec == "f64" else np.float32
+    comm = gpu_util.comm_for(2)
     for sides in ([(64, 64), (4, 4), (20, 30), (16, 16), (7, 9), (96, 80)], [(8, 8), (30, 18)]):
         work = []
         for i in range(24):
@@ -71,7 +74,7 @@ def test_noalloc_planes_and_tiny_planes(prec):
             x = random_input(spec, i)
             a, b = (P.DeviceBuffer(x.size * np.dtype(rdt).itemsize) for _ in range(2))
             a.upload(x.astype(rdt))
-            pl = P.Plan("c2c", spec.n, a.ptr, b.ptr, sign=spec.sign, comm=comm_for(2), prec=prec)
+            pl = P.Plan("c2c", spec.n, a.ptr, b.ptr, sign=spec.sign, comm=comm, prec=prec)
             assert pl.ok
             work.append((spec, x, a, b, pl))
         assert P.execute_batch_noalloc([w[4] for w in work]) == 0

@@ -8,6 +8,7 @@ import pytest
 import pfft_amd as P
 from gpu_util import spec_of, random_input, run_gpu, oracle_out, rel_l2
 from test_gpu_tune import _plan_lines, tune_all   # noqa: F401 (fixture)
+from shared_comm import shared_comm   # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 TO, TI = P.TRANSPOSED_OUT, P.TRANSPOSED_IN

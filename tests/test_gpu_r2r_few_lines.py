@@ -5,9 +5,11 @@ import time
 
 import pytest
 
+import gpu_util
 import pfft_amd as P
-from gpu_util import spec_of, random_input, run_gpu, oracle_out, rel_l2, comm_for
+from gpu_util import spec_of, random_input, run_gpu, oracle_out, rel_l2
 from test_gpu_mixed import KINDS
+from shared_comm import shared_comm   # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -17,7 +19,7 @@ def plan_us(n, kind, prec, howmany):
     for v in n:
         size *= v
     a, b = P.DeviceBuffer(size), P.DeviceBuffer(size)
-    plan = P.Plan("r2r", n, a.ptr, b.ptr, howmany=howmany, comm=comm_for(1), prec=prec,
+    plan = P.Plan("r2r", n, a.ptr, b.ptr, howmany=howmany, comm=gpu_util.comm_for(1), prec=prec,
                   kinds=[KINDS[kind]] * len(n), flags=P.ESTIMATE)
     assert plan.ok
     best = 1e9

@@ -6,8 +6,10 @@ in a batch."""
 import numpy as np
 import pytest
 
+import gpu_util
 import pfft_amd as P
-from gpu_util import spec_of, random_input, oracle_out, rel_l2, comm_for, n_scalars
+from gpu_util import spec_of, random_input, oracle_out, rel_l2, n_scalars
+from shared_comm import shared_comm   # noqa: F401 (fixture)
 
 pytestmark = pytest.mark.gpu
 TI, TO = P.TRANSPOSED_IN, P.TRANSPOSED_OUT
@@ -36,7 +38,7 @@ def plan_and_buffers(case, prec, seed):
     a, b = P.DeviceBuffer(nin * x.itemsize), P.DeviceBuffer((nout + guard) * x.itemsize)
     a.upload(x)
     b.upload(np.full(nout + guard, 7.0, rdt))
-    pl = P.Plan("r2r", n, a.ptr, b.ptr, ni, no, howmany, 0, flags, comm=comm_for(rnk_pm),
+    pl = P.Plan("r2r", n, a.ptr, b.ptr, ni, no, howmany, 0, flags, comm=gpu_util.comm_for(rnk_pm),
                 skip=skip, prec=prec, kinds=K[:len(n)])
     assert pl.ok
     return spec, x, a, b, pl, nout, rdt
