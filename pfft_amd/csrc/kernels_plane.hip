@@ -6,13 +6,12 @@ namespace pfk {
 // Resident workgroups walk the planes.
 template <typename T>
 __global__ void __launch_bounds__(1024)
-k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const T *__restrict__ src,
-        T *__restrict__ dst) {
+k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const int last,
+        const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char plane_smem[];
   stamp_begin(P, blockIdx.x);
   bool tables = true;
-  int64_t id = blockIdx.x;
-  for (; id < nplanes; id += gridDim.x, tables = false) {
+  for (int64_t id = blockIdx.x; id < nplanes; id += gridDim.x, tables = false) {
     int64_t u = id, s = 0, d = 0;
     for (int i = 0; i < P.nb; ++i) {
       const int64_t k = u % P.bext[i];
@@ -22,7 +21,7 @@ k_plane(const pfk_pass P, const PlaneGeo G, const int64_t nplanes, const T *__re
     }
     plane_tile<T>(G, P.sign, src + 2 * s, dst + 2 * d, P.twm, G.twc, tables, plane_smem);
   }
-  stamp_end(P, nplanes - 1 - (id - gridDim.x));
+  stamp_end(P, walk_left(last));
 }
 
 static size_t plane_lds(const pfk_pass *p, PlaneGeo *g) {
@@ -116,7 +115,7 @@ static int launch_plane_t(const pfk_pass *p, const PlaneGeo &g, int nt, size_t l
   if (per > 16 / (nt / 64)) per = 16 / (nt / 64);
   const int64_t res = per * ncu, grid = planes < res ? planes : res;
   hipLaunchKernelGGL(k_plane<T>, dim3((unsigned)grid), dim3(nt), lds, g_stream, *p, g, planes,
-                     (const T *)src, (T *)dst);
+                     (int)((planes - 1) % grid), (const T *)src, (T *)dst);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_launch_pass(plane)", e); return 1; }
   return 0;

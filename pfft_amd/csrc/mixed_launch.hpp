@@ -10,17 +10,16 @@ namespace pfk {
 template <typename T, int KIND, bool BIG>
 __global__ void __launch_bounds__(512, 4)
 k_mixed(const pfk_pass P, const MixGeo G, const int64_t ntiles, const int64_t nlines,
-        const T *__restrict__ src, T *__restrict__ dst) {
+        const int last, const T *__restrict__ src, T *__restrict__ dst) {
   extern __shared__ unsigned char mix_smem[];
   stamp_begin(P, blockIdx.x);
   mix_table<T>(P, G, mix_smem);
   int odd = 0;
-  int64_t id = blockIdx.x;
-  for (; id < ntiles; id += gridDim.x, odd ^= 1) {
+  for (int64_t id = blockIdx.x; id < ntiles; id += gridDim.x, odd ^= 1) {
     const int64_t tile = P.xcd_remap ? xcd_remap(id, ntiles) : id;
     mixed_tile<T, KIND, BIG>(P, G, tile * G.C, nlines, odd, src, dst, mix_smem);
   }
-  stamp_end(P, ntiles - 1 - (id - gridDim.x));
+  stamp_end(P, walk_left(last));
 }
 
 // Launch with nt threads and `lds` bytes of LDS per workgroup.
@@ -53,7 +52,7 @@ static int launch_mixed_k(const pfk_pass *p, const MixGeo &g, int nt, size_t lds
   if (per_cu < 1) per_cu = 1;
   const int64_t res = per_cu * (ncu / 8) * 8, grid = ntiles < res ? ntiles : res;
   hipLaunchKernelGGL((k_mixed<T, KIND, BIG>), dim3((unsigned)grid), dim3(nt), lds, g_stream, *p, g,
-                     ntiles, lines, (const T *)src, (T *)dst);
+                     ntiles, lines, (int)((ntiles - 1) % grid), (const T *)src, (T *)dst);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) { set_error("pfk_launch_pass(mixed)", e); return -1; }
   return 0;

@@ -41,6 +41,15 @@ __device__ __forceinline__ void stamp_end(const pfk_pass &P, const int64_t left)
   if (P.stamp_end && left < PFK_STAMP_ENDS) P.stamp_end[left] = wall_clock64();
 }
 
+// `left` of this workgroup in a walk whose last item workgroup `last` runs.  From
+// the block index rather than the walk's counter, whose life to the end of the
+// kernel cost the mixed-radix kernel a spilled register (100^3 complex128 47.9 ->
+// 49.5 us).
+__device__ __forceinline__ int64_t walk_left(const int last) {
+  const int left = last - (int)blockIdx.x;
+  return left < 0 ? left + (int)gridDim.x : left;
+}
+
 extern hipStream_t g_stream;
 extern int g_generic_only;   // PFFT_AMD_GENERIC_ONLY=1: route every pass to the general kernel
 extern int g_max_lds;
