@@ -428,9 +428,10 @@ void pfft_execute_batch(const pfft_plan *plans, int count);
  * (code under graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  Same kernels and result
  * as pfft_execute_batch (launched directly, not through a graph), with the
- * work-list in a fixed device array of the library (1.1 MiB, 2048 task
- * records of 560 bytes, per GPU, kept until the process ends): at most 2048 passes in total (a 3-d plan has 3), plans of
- * one precision (pfft_plan or pfftf_plan handles) on device arrays, and no
+ * work-list in a fixed device array of the library (1.7 MiB: 2048 task
+ * records of 608 bytes and as many plane geometries of 256, per GPU, kept
+ * until the process ends): at most 2048 passes in total (a 3-d plan has 3),
+ * plans of one precision (pfft_plan or pfftf_plan handles) on device arrays, and no
  * long-line, r2r or MFMA-form passes.  Blocking; returns 0 on success and 1
  * with a message otherwise.  Calls that overlap on one GPU share the array
  * and race. */

@@ -19,7 +19,8 @@
 // Only the forward table exists: a backward transform conjugates its input and
 // its output.
 //
-// Primes above 13 (one stage each, radix R): with x_0 apart, the pair sums
+// Primes above 13 (one stage each, radix R; up to 587 in complex128 and 1181 in
+// complex64, where eight lines in two tiles fill LDS): with x_0 apart, the pair sums
 // A_r = x_r + x_(R-r) and differences B_r = x_r - x_(R-r), r <= (R-1)/2, give
 //   Y_q     = x_0 + sum_r cos(2 pi q r/R) A_r - i sum_r sin(2 pi q r/R) B_r,
 //   Y_(R-q) = the same with + i,
@@ -32,13 +33,16 @@
 // their own those steps were two further sweeps: 256^3 complex128 DCT-II and
 // DCT-III 1218 -> 578 us, 87-96 us a pass.
 //
-// Bound: the HBM sweep, at 3.7-5.1 TB/s (0.7-1.5 for the general kernel, whose
-// stages sum each output over its radix with a division per element).
-// Forward+backward pairs, general kernel -> this one: c2c 360x300x250
-// complex128 4.26 -> 1.28 ms, r2c 210x196x330 complex64 908 -> 210 us, c2c
-// 29x27x31 complex128 142 -> 96 us.  Without any stage arithmetic and
-// exchanges the first of these takes 1.07 ms.  Registers (128) and LDS leave
-// 16 waves per CU in flight.
+// Bound: the complex passes by waiting, 3.7-5.1 TB/s with 9-14 waves per CU and the
+// vector units 25-42% busy (loads, exchanges and stores of a tile follow one
+// another; rows that are not whole segments are read up to 1.9 times); the
+// single-precision real and the r2r lines by vector instructions, 70% busy, the
+// latter at 2.8-3.0 TB/s.  The general kernel, whose stages sum each output over
+// its radix with a division per element, runs at 0.7-1.5 TB/s.  Forward+backward
+// pairs, general kernel -> this one: c2c 360x300x250 complex128 4.26 -> 1.28 ms,
+// r2c 210x196x330 complex64 908 -> 210 us, c2c 29x27x31 complex128 142 -> 96 us.
+// Without any stage arithmetic and exchanges the first of these takes 1.07 ms.
+// Registers (128) and LDS leave 16 waves per CU in flight.
 #pragma once
 #include "dft_regs.hpp"
 
